@@ -66,6 +66,36 @@ int sc_qmm_bf16(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, c
                 int group_size, void *hip_stream);
 
 /*
+ * Workspace variants, for products of many rows: with a workspace of at least
+ * sc_qmm_workspace_bytes(M, N, K) bytes (16-byte aligned, overlapping no other
+ * argument) the weights are dequantized into it once per call and a dense bf16 GEMM
+ * reads them, instead of every 256-row tile dequantizing its own copy.  The function
+ * returns 0 for shapes where that is not the faster; with a null, smaller or
+ * misaligned workspace the call is the one without the suffix.  The weights are
+ * rounded to bf16 alike on both; the fp32 sums run in another order.  The workspace
+ * holds nothing between calls and may be reused once the call's work on the stream is
+ * done.  Other arguments, results and reference call sites as without the suffix.
+ */
+int64_t sc_qmm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int sc_qmm_bf16_ws(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
+                   const uint16_t *bias_or_null, uint16_t *y, int64_t M, int64_t N, int64_t K, int bits,
+                   int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream);
+int sc_qmm_rmsnorm_bf16_ws(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight, float eps,
+                           uint16_t *h_out_or_null, uint16_t *xn_out, const uint32_t *wq, const uint16_t *scales,
+                           const uint16_t *biases, const uint16_t *bias_or_null, uint16_t *y, int64_t M, int64_t N,
+                           int64_t K, int bits, int group_size, void *workspace_or_null, int64_t workspace_bytes,
+                           void *hip_stream);
+int sc_qmm_add_rmsnorm_bf16_ws(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
+                               const uint16_t *bias_or_null, const uint16_t *residual, const uint16_t *norm_weight,
+                               float eps, uint16_t *h_out, uint16_t *xn_out, int64_t M, int64_t N, int64_t K, int bits,
+                               int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream);
+int sc_qmm_swiglu_bf16_ws(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight_or_null,
+                          float eps, uint16_t *h_out_or_null, uint16_t *xn_out_or_null, const uint32_t *wq,
+                          const uint16_t *scales, const uint16_t *biases, const uint16_t *bias_or_null,
+                          uint16_t *act_out, uint16_t *gate_up_scratch, int64_t M, int64_t I, int64_t K, int bits,
+                          int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream);
+
+/*
  * sc_qmm_bf16 with an explicit kernel choice (SC_QMM_PATH_*): lets tests and
  * benchmarks run both kernels on the same shape.  Same reference call sites.
  */

@@ -22,6 +22,11 @@ EXPORTS = (
     "sc_abi_version",
     "sc_last_error",
     "sc_qmm_bf16",
+    "sc_qmm_workspace_bytes",
+    "sc_qmm_bf16_ws",
+    "sc_qmm_rmsnorm_bf16_ws",
+    "sc_qmm_add_rmsnorm_bf16_ws",
+    "sc_qmm_swiglu_bf16_ws",
     "sc_qmm_bf16_path",
     "sc_qmm_bf16_noalloc",
     "sc_qmm_bf16_band",
@@ -83,6 +88,10 @@ def load():
         lib.sc_last_error.restype = ctypes.c_char_p
         lib.sc_qmm_bf16.argtypes = [p, p, p, p, p, p, i64, i64, i64, i32, i32, p]
         lib.sc_qmm_bf16.restype = i32
+        lib.sc_qmm_workspace_bytes.argtypes = [i64, i64, i64]
+        lib.sc_qmm_workspace_bytes.restype = i64
+        lib.sc_qmm_bf16_ws.argtypes = [p, p, p, p, p, p, i64, i64, i64, i32, i32, p, i64, p]
+        lib.sc_qmm_bf16_ws.restype = i32
         lib.sc_qmm_bf16_path.argtypes = [p, p, p, p, p, p, i64, i64, i64, i32, i32, i32, p]
         lib.sc_qmm_bf16_path.restype = i32
         lib.sc_qmm_bf16_noalloc.argtypes = [p, p, p, p, p, p, i64, i64, i64, i32, i32, p]
@@ -100,13 +109,19 @@ def load():
         f32 = ctypes.c_float
         lib.sc_qmm_rmsnorm_bf16.argtypes = [p, p, p, f32, p, p, p, p, p, p, p, i64, i64, i64, i32, i32, p]
         lib.sc_qmm_rmsnorm_bf16.restype = i32
+        lib.sc_qmm_rmsnorm_bf16_ws.argtypes = [p, p, p, f32, p, p, p, p, p, p, p, i64, i64, i64, i32, i32, p, i64, p]
+        lib.sc_qmm_rmsnorm_bf16_ws.restype = i32
         lib.sc_qmm_add_rmsnorm_bf16.argtypes = [p, p, p, p, p, p, p, f32, p, p, i64, i64, i64, i32, i32, p]
         lib.sc_qmm_add_rmsnorm_bf16.restype = i32
+        lib.sc_qmm_add_rmsnorm_bf16_ws.argtypes = [p, p, p, p, p, p, p, f32, p, p, i64, i64, i64, i32, i32, p, i64, p]
+        lib.sc_qmm_add_rmsnorm_bf16_ws.restype = i32
         lib.sc_decode_head_bf16.argtypes = [p, p, p, f32, p, p, p, p, p, p, p, i64, i64, i64, i32, i32, p, p, i64,
                                             i64, p, p, i64, p, i64, p]
         lib.sc_decode_head_bf16.restype = i32
         lib.sc_qmm_swiglu_bf16.argtypes = [p, p, p, f32, p, p, p, p, p, p, p, p, i64, i64, i64, i32, i32, p]
         lib.sc_qmm_swiglu_bf16.restype = i32
+        lib.sc_qmm_swiglu_bf16_ws.argtypes = [p, p, p, f32, p, p, p, p, p, p, p, p, i64, i64, i64, i32, i32, p, i64, p]
+        lib.sc_qmm_swiglu_bf16_ws.restype = i32
         lib.sc_rms_norm_bf16.argtypes = [p, p, p, p, p, i64, i64, f32, p]
         lib.sc_rms_norm_bf16.restype = i32
         lib.sc_rope_append_kv_bf16.argtypes = [p, i64, i64, i64, i64, i64, i64, p, p, i64, p, p, i64, p, i64, p]
@@ -191,6 +206,21 @@ def _bf16(t, name):
     return t
 
 
+def _qmm_workspace(M, N, K, device):
+    """(tensor, bytes) of the workspace a product of M rows runs faster with, from the
+    current stream's caching allocator, or (None, 0): small products, and when the
+    allocation fails the product runs without."""
+    if M < 1024:        # the library wants none for fewer rows
+        return None, 0
+    n = load().sc_qmm_workspace_bytes(M, N, K)
+    if n <= 0:
+        return None, 0
+    try:
+        return torch.empty(n, dtype=torch.uint8, device=device), n
+    except torch.cuda.OutOfMemoryError:
+        return None, 0
+
+
 def qmm(x, wq, scales, biases, bias=None, bits=4, group_size=64, path=PATH_AUTO, out=None, no_alloc=False,
         band_plan=None):
     """y = bf16(x @ dequant(wq, scales, biases)^T) (+ bias), x [..., K] -> [..., N].
@@ -238,6 +268,10 @@ def qmm(x, wq, scales, biases, bias=None, bits=4, group_size=64, path=PATH_AUTO,
             raise ValueError("the allocation-free entry point chooses its kernel itself (path must be AUTO)")
         rc = lib.sc_qmm_bf16_noalloc(_ptr(x2), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(y),
                                      M, N, K, bits, group_size, st)
+    elif path == PATH_AUTO:
+        ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
+        rc = lib.sc_qmm_bf16_ws(_ptr(x2), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(y),
+                                M, N, K, bits, group_size, _ptr(ws), ws_bytes, st)
     else:
         rc = lib.sc_qmm_bf16_path(_ptr(x2), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(y),
                                   M, N, K, bits, group_size, path, st)
@@ -293,9 +327,10 @@ def qmm_rmsnorm(x, norm_weight, eps, wq, scales, biases, residual=None, h_out=No
     xn = xn_out if xn_out is not None else torch.empty((M, K), dtype=torch.bfloat16, device=x.device)
     _rows(xn, K, "xn_out")
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    rc = lib.sc_qmm_rmsnorm_bf16(_ptr(x), _ptr(residual), _ptr(norm_weight.contiguous()), float(eps), _ptr(h_out),
-                                 _ptr(xn), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(y), M, N, K, bits,
-                                 group_size, _stream(x))
+    ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
+    rc = lib.sc_qmm_rmsnorm_bf16_ws(_ptr(x), _ptr(residual), _ptr(norm_weight.contiguous()), float(eps), _ptr(h_out),
+                                    _ptr(xn), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(y), M, N, K,
+                                    bits, group_size, _ptr(ws), ws_bytes, _stream(x))
     _check(rc, "sc_qmm_rmsnorm_bf16")
     return y.reshape(*lead, N), xn.reshape(*lead, K)
 
@@ -322,9 +357,10 @@ def qmm_add_rmsnorm(x, wq, scales, biases, residual, norm_weight, eps, bias=None
     xn = xn_out if xn_out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _rows(h, N, "h_out")
     _rows(xn, N, "xn_out")
-    rc = lib.sc_qmm_add_rmsnorm_bf16(_ptr(x), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(residual),
-                                     _ptr(norm_weight.contiguous()), float(eps), _ptr(h), _ptr(xn), M, N, K, bits,
-                                     group_size, _stream(x))
+    ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
+    rc = lib.sc_qmm_add_rmsnorm_bf16_ws(_ptr(x), _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(residual),
+                                        _ptr(norm_weight.contiguous()), float(eps), _ptr(h), _ptr(xn), M, N, K, bits,
+                                        group_size, _ptr(ws), ws_bytes, _stream(x))
     _check(rc, "sc_qmm_add_rmsnorm_bf16")
     return h.reshape(*lead, N), xn.reshape(*lead, N)
 
@@ -409,9 +445,10 @@ def qmm_swiglu(x, wq, scales, biases, norm_weight=None, eps=1e-5, residual=None,
     gu = gate_up_scratch if gate_up_scratch is not None else torch.empty((M, N), dtype=torch.bfloat16,
                                                                           device=x.device)
     _rows(gu, N, "gate_up_scratch")
-    rc = lib.sc_qmm_swiglu_bf16(_ptr(x), _ptr(residual), _ptr(norm_weight), float(eps), _ptr(h_out), _ptr(xn),
-                                _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(act), _ptr(gu), M, I, K, bits,
-                                group_size, _stream(x))
+    ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
+    rc = lib.sc_qmm_swiglu_bf16_ws(_ptr(x), _ptr(residual), _ptr(norm_weight), float(eps), _ptr(h_out), _ptr(xn),
+                                   _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(act), _ptr(gu), M, I, K,
+                                   bits, group_size, _ptr(ws), ws_bytes, _stream(x))
     _check(rc, "sc_qmm_swiglu_bf16")
     return act.reshape(*lead, I), (xn.reshape(*lead, K) if xn is not None else None)
 

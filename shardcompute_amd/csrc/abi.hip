@@ -24,6 +24,10 @@ int launch_qgemv_skinny(const uint16_t *x, const uint32_t *wq, const uint16_t *s
 int launch_qgemm_mfma(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                       int swiglu_half = 0, bool no_alloc = false);
+int64_t qgemm_dense_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
+                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
+                       int swiglu_half, void *ws, int64_t ws_bytes);
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                       bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr);
@@ -177,12 +181,24 @@ static bool band_first(int64_t M, int64_t N, int64_t K) {
     return M > 16 || (M > 8 && (K > 4096 || N <= 8192));
 }
 
+// The caller's workspace of a call (none: ws null), for the products whose weights are
+// dequantized once per call (qgemm_dense.hip).
+struct QmmWorkspace {
+    void *ws = nullptr;
+    int64_t bytes = 0;
+};
+
 static int qmm_dispatch(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                         const uint16_t *bias, uint16_t *y, int64_t M, int64_t N, int64_t K, int bits,
-                        int group_size, void *stream, int path, bool no_alloc = false, SplitKeep *keep = nullptr) {
+                        int group_size, void *stream, int path, bool no_alloc = false, SplitKeep *keep = nullptr,
+                        QmmWorkspace wsp = {}) {
     int rc = check_qmm(x, wq, s, b, y, M, N, K, bits, group_size);
     if (rc) return rc;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (path == SC_QMM_PATH_AUTO && wsp.ws) {
+        rc = launch_qgemm_dense(x, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, 0, wsp.ws, wsp.bytes);
+        if (rc != SC_EUNSUPPORTED) return rc;
+    }
     if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
                                                                                     : SC_QMM_PATH_GEMM;
     if (path == SC_QMM_PATH_BAND) {
@@ -228,8 +244,8 @@ static bool overlap(const void *a, size_t an, const void *b, size_t bn) {
 static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw, float eps, uint16_t *h_out,
                      uint16_t *x_out, const uint32_t *wq, const uint16_t *s, const uint16_t *b, const uint16_t *bias,
                      uint16_t *y, int64_t M, int64_t N, int64_t K, int bits, int group_size, void *stream,
-                     int64_t swiglu_half, uint16_t *gu_scratch, const HeadArgmax *head = nullptr,
-                     bool *head_done = nullptr) {
+                     int64_t swiglu_half, uint16_t *gu_scratch, QmmWorkspace wsp = {},
+                     const HeadArgmax *head = nullptr, bool *head_done = nullptr) {
     const char *what = swiglu_half ? "qmm_swiglu" : "qmm_rmsnorm";
     const uint16_t *xin = nw ? x_out : x;
     int rc = check_qmm(xin, wq, s, b, y, M, N, K, bits, group_size);
@@ -277,7 +293,14 @@ static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw,
         rc = launch_rms_norm(x, res, nw, x_out, res ? h_out : nullptr, M, K, eps, st);
         if (rc) return rc;
     }
-    if (!swiglu_half) return qmm_dispatch(xin, wq, s, b, bias, y, M, N, K, bits, group_size, stream, SC_QMM_PATH_AUTO);
+    if (!swiglu_half)
+        return qmm_dispatch(xin, wq, s, b, bias, y, M, N, K, bits, group_size, stream, SC_QMM_PATH_AUTO, false,
+                            nullptr, wsp);
+    if (wsp.ws) {
+        rc = launch_qgemm_dense(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, (int)swiglu_half, wsp.ws,
+                                wsp.bytes);
+        if (rc != SC_EUNSUPPORTED) return rc;
+    }
     if (band_first(M, N, K)) {
         // the band kernel's split-K pass applies silu(gate) * up itself
         rc = launch_qgemm_band(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half, 0,
@@ -314,6 +337,15 @@ int sc_qmm_bf16(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, c
                 int group_size, void *hip_stream) {
     return qmm_dispatch(x, wq, scales, biases, bias_or_null, y, M, N, K, bits, group_size, hip_stream,
                         SC_QMM_PATH_AUTO);
+}
+
+int64_t sc_qmm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return qgemm_dense_workspace_bytes(M, N, K); }
+
+int sc_qmm_bf16_ws(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
+                   const uint16_t *bias_or_null, uint16_t *y, int64_t M, int64_t N, int64_t K, int bits,
+                   int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream) {
+    return qmm_dispatch(x, wq, scales, biases, bias_or_null, y, M, N, K, bits, group_size, hip_stream,
+                        SC_QMM_PATH_AUTO, false, nullptr, {workspace_or_null, workspace_bytes});
 }
 
 int sc_qmm_bf16_path(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
@@ -494,19 +526,28 @@ int sc_decode_plan_read_trace(void *plan, uint32_t *stamps, int64_t n, int *work
 
 void sc_decode_plan_destroy(void *plan) { decode_plan_destroy(plan); }
 
+int sc_qmm_rmsnorm_bf16_ws(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight, float eps,
+                           uint16_t *h_out_or_null, uint16_t *xn_out, const uint32_t *wq, const uint16_t *scales,
+                           const uint16_t *biases, const uint16_t *bias_or_null, uint16_t *y, int64_t M, int64_t N,
+                           int64_t K, int bits, int group_size, void *workspace_or_null, int64_t workspace_bytes,
+                           void *hip_stream) {
+    if (!norm_weight || !xn_out) return set_error(SC_EINVAL, "qmm_rmsnorm: null pointer argument");
+    return qmm_fused(x, residual_or_null, norm_weight, eps, h_out_or_null, xn_out, wq, scales, biases, bias_or_null, y,
+                     M, N, K, bits, group_size, hip_stream, 0, nullptr, {workspace_or_null, workspace_bytes});
+}
+
 int sc_qmm_rmsnorm_bf16(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight, float eps,
                         uint16_t *h_out_or_null, uint16_t *xn_out, const uint32_t *wq, const uint16_t *scales,
                         const uint16_t *biases, const uint16_t *bias_or_null, uint16_t *y, int64_t M, int64_t N,
                         int64_t K, int bits, int group_size, void *hip_stream) {
-    if (!norm_weight || !xn_out) return set_error(SC_EINVAL, "qmm_rmsnorm: null pointer argument");
-    return qmm_fused(x, residual_or_null, norm_weight, eps, h_out_or_null, xn_out, wq, scales, biases, bias_or_null, y,
-                     M, N, K, bits, group_size, hip_stream, 0, nullptr);
+    return sc_qmm_rmsnorm_bf16_ws(x, residual_or_null, norm_weight, eps, h_out_or_null, xn_out, wq, scales, biases,
+                                  bias_or_null, y, M, N, K, bits, group_size, nullptr, 0, hip_stream);
 }
 
-int sc_qmm_add_rmsnorm_bf16(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
-                            const uint16_t *bias_or_null, const uint16_t *residual, const uint16_t *norm_weight,
-                            float eps, uint16_t *h_out, uint16_t *xn_out, int64_t M, int64_t N, int64_t K, int bits,
-                            int group_size, void *hip_stream) {
+int sc_qmm_add_rmsnorm_bf16_ws(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
+                               const uint16_t *bias_or_null, const uint16_t *residual, const uint16_t *norm_weight,
+                               float eps, uint16_t *h_out, uint16_t *xn_out, int64_t M, int64_t N, int64_t K, int bits,
+                               int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream) {
     int rc = check_qmm(x, wq, scales, biases, xn_out, M, N, K, bits, group_size);
     if (rc) return rc;
     if (!residual || !norm_weight || !h_out) return set_error(SC_EINVAL, "qmm_add_rmsnorm: null pointer argument");
@@ -523,11 +564,19 @@ int sc_qmm_add_rmsnorm_bf16(const uint16_t *x, const uint32_t *wq, const uint16_
     // writes its rows itself writes them into xn_out, which the pass then reads
     SplitKeep keep;
     rc = qmm_dispatch(x, wq, scales, biases, bias_or_null, xn_out, M, N, K, bits, group_size, hip_stream,
-                      SC_QMM_PATH_AUTO, false, &keep);
+                      SC_QMM_PATH_AUTO, false, &keep, {workspace_or_null, workspace_bytes});
     if (rc) return rc;
     return launch_split_add_rms_norm(keep.partials, keep.splits, xn_out, keep.splits ? bias_or_null : nullptr,
                                      residual, norm_weight, h_out, xn_out, M, N, eps,
                                      reinterpret_cast<hipStream_t>(hip_stream));
+}
+
+int sc_qmm_add_rmsnorm_bf16(const uint16_t *x, const uint32_t *wq, const uint16_t *scales, const uint16_t *biases,
+                            const uint16_t *bias_or_null, const uint16_t *residual, const uint16_t *norm_weight,
+                            float eps, uint16_t *h_out, uint16_t *xn_out, int64_t M, int64_t N, int64_t K, int bits,
+                            int group_size, void *hip_stream) {
+    return sc_qmm_add_rmsnorm_bf16_ws(x, wq, scales, biases, bias_or_null, residual, norm_weight, eps, h_out,
+                                      xn_out, M, N, K, bits, group_size, nullptr, 0, hip_stream);
 }
 
 int sc_decode_head_bf16(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight, float eps,
@@ -553,11 +602,22 @@ int sc_decode_head_bf16(const uint16_t *x, const uint16_t *residual_or_null, con
                   ids, tokens_or_null, (long)tokens_cols, step_or_null, counters_or_null, (int)n_counters};
     bool done = false;
     int rc = qmm_fused(x, residual_or_null, norm_weight, eps, h_out_or_null, xn_out, wq, scales, biases, bias_or_null,
-                       logits, M, N, K, bits, group_size, hip_stream, 0, nullptr, M == 1 ? &hd : nullptr, &done);
+                       logits, M, N, K, bits, group_size, hip_stream, 0, nullptr, {}, M == 1 ? &hd : nullptr, &done);
     if (rc || done) return rc;
     rc = launch_argmax(logits, M, N, ids, tokens_or_null, tokens_stride, tokens_cols, step_or_null, st);
     if (rc || !n_counters) return rc;
     return launch_add_i32(counters_or_null, n_counters, 1, st);
+}
+
+int sc_qmm_swiglu_bf16_ws(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight_or_null,
+                          float eps, uint16_t *h_out_or_null, uint16_t *xn_out_or_null, const uint32_t *wq,
+                          const uint16_t *scales, const uint16_t *biases, const uint16_t *bias_or_null,
+                          uint16_t *act_out, uint16_t *gate_up_scratch, int64_t M, int64_t I, int64_t K, int bits,
+                          int group_size, void *workspace_or_null, int64_t workspace_bytes, void *hip_stream) {
+    if (norm_weight_or_null && !xn_out_or_null) return set_error(SC_EINVAL, "qmm_swiglu: xn_out required with a norm");
+    return qmm_fused(x, residual_or_null, norm_weight_or_null, eps, h_out_or_null, xn_out_or_null, wq, scales, biases,
+                     bias_or_null, act_out, M, 2 * I, K, bits, group_size, hip_stream, I, gate_up_scratch,
+                     {workspace_or_null, workspace_bytes});
 }
 
 int sc_qmm_swiglu_bf16(const uint16_t *x, const uint16_t *residual_or_null, const uint16_t *norm_weight_or_null,
@@ -565,9 +625,8 @@ int sc_qmm_swiglu_bf16(const uint16_t *x, const uint16_t *residual_or_null, cons
                        const uint16_t *scales, const uint16_t *biases, const uint16_t *bias_or_null, uint16_t *act_out,
                        uint16_t *gate_up_scratch, int64_t M, int64_t I, int64_t K, int bits, int group_size,
                        void *hip_stream) {
-    if (norm_weight_or_null && !xn_out_or_null) return set_error(SC_EINVAL, "qmm_swiglu: xn_out required with a norm");
-    return qmm_fused(x, residual_or_null, norm_weight_or_null, eps, h_out_or_null, xn_out_or_null, wq, scales, biases,
-                     bias_or_null, act_out, M, 2 * I, K, bits, group_size, hip_stream, I, gate_up_scratch);
+    return sc_qmm_swiglu_bf16_ws(x, residual_or_null, norm_weight_or_null, eps, h_out_or_null, xn_out_or_null, wq,
+                                 scales, biases, bias_or_null, act_out, gate_up_scratch, M, I, K, bits, group_size, nullptr, 0, hip_stream);
 }
 
 

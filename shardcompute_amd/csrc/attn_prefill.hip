@@ -19,26 +19,27 @@ namespace sc {
 namespace {
 
 // Causal GQA attention of many new positions (the same contraction as attn_kernel,
-// attention.py:437-466), for head_dim 128: a workgroup owns 128 query columns, the
+// attention.py:437-466), for head_dim 128 and 64: a workgroup owns 128 query columns, the
 // R query heads of kv head hk at positions [PB qb, PB qb + PB) (PB = 128 / R; column
 // c is position PB qb + c / R, head hk R + c % R), so each 64-key block of K and Vt
 // staged in LDS serves 128 columns (attn_kernel's workgroups serve 16).  4 waves,
 // wave w owns columns [32 w, 32 w + 32), on v_mfma_f32_32x32x16_bf16:
-// * S^T[64 keys x 32 columns] = K Q^T: two 32-key blocks, 8 k-steps of 16 dims; the
+// * S^T[64 keys x 32 columns] = K Q^T: two 32-key blocks, D / 16 k-steps of 16 dims; the
 //   column's q is operand B (registers, loaded once); operand A row i is key
 //   swap23(i) (bits 2 and 3 of i exchanged), so that accumulator register r of lane
 //   (column li, half lh) holds key 16 (r / 8) + 8 lh + r % 8 of the 32-key block:
 //   every 8 registers are 8 consecutive keys;
 // * online softmax per column over its 32 values and the partner lane li + 32, with
-//   scores kept unscaled (one FMA folds the scale into the exponent); the running
-//   maximum is only moved when it grew by more than 2^8 in probability, so that O
-//   is rescaled in few blocks (probabilities stay below 256, exact in the ratio);
+//   scores kept unscaled (one FMA folds the scale into the exponent); with head_dim 128
+//   the running maximum is only moved when it grew by more than 2^8 in probability, so
+//   that O is rescaled in few blocks (probabilities stay below 256, exact in the ratio);
 //   keys are masked only in the blocks that reach a column's last key;
-// * O^T[128 dims x 32 columns] += Vt P^T in 4 k-steps of 16 keys: P^T is operand B
+// * O^T[D dims x 32 columns] += Vt P^T in 4 k-steps of 16 keys: P^T is operand B
 //   straight from the S^T registers (bf16), operand A one 16-byte read of 8
 //   consecutive keys of a Vt row;
 // * K and Vt blocks reach LDS by LDS-DMA, one block ahead in a 2-stage ring (64 KB,
-//   so that two workgroups, 8 waves, share a CU and hide each other's waits), their
+//   so that two workgroups, 8 waves, share a CU and hide each other's waits; head_dim 64:
+//   32 KB and 168 registers, three workgroups), their
 //   16-byte chunks XOR-swizzled by row so that every operand read is conflict-free;
 // * cache slots past the length may hold anything, NaN included: their scores are
 //   masked and, in the block that crosses the length, their V pieces are zeroed
@@ -47,13 +48,24 @@ namespace {
 //   rounds in heavy/light pairs.
 // The result is bf16(O / l) per column, as attn_kernel writes it (P in bf16, fp32
 // sums), with the sums in another order.
-constexpr int FA_COLS = 128, FA_KB = 64, FA_D = 128, FA_THREADS = 256;
-constexpr int FA_KTILE = FA_KB * FA_D * 2;           // 16 KB: 64 keys x 256 B
-constexpr int FA_VTILE = FA_D * FA_KB * 2;           // 16 KB: 128 dims x 128 B
-constexpr int FA_STAGE = FA_KTILE + FA_VTILE;
+constexpr int FA_COLS = 128, FA_KB = 64, FA_THREADS = 256;
 constexpr int FA_NST = 2;                            // LDS stages: block blk being read, blk + 1 landing
-constexpr int FA_LDS = FA_NST * FA_STAGE;            // 64 KB
 constexpr int FA_SAHEAD = 4;                         // operand reads in flight ahead of the MFMAs
+template <int D>
+struct FaGeo {
+    static constexpr int KROW = D * 2;                           // bytes of a key row (256 or 128)
+    static constexpr int KTILE = FA_KB * KROW, VTILE = D * FA_KB * 2;
+    static constexpr int STAGE = KTILE + VTILE;                  // 32 or 16 KB
+    static constexpr int LDS = FA_NST * STAGE;                   // 64 or 32 KB
+    static constexpr int KSTEPS = D / 16;                        // 16-dim steps of S^T
+    static constexpr int DB = D / 32;                            // 32-dim blocks of O^T
+    static constexpr int KROWS_PI = 1024 / KROW;                 // key rows of a DMA instruction
+    static constexpr int DMA = KTILE / 1024 / 4;                 // K (and Vt) DMA instructions per wave
+    // the growth of a column's maximum (log2) that moves it.  head_dim 64 rescales few
+    // registers and always moves it: the largest probabilities then lie just below 1, where
+    // bf16 rounds them best, as in attn_kernel (2-10 % less error than with 8, 4 % slower)
+    static constexpr float LAZY = D == 64 ? 0.f : 8.f;
+};
 
 struct FaArgs {
     const uint16_t *q;
@@ -78,8 +90,14 @@ __device__ __forceinline__ int fa_swap23(int i) { return (i & ~12) | ((i & 4) <<
 // byte offset of 16-byte chunk c of K tile row r (16 chunks a row): chunk c of key row
 // r sits at position c ^ swap23(r) % 16, so the rows swap23(i), i = 0..15, that lanes
 // 0..15 of an operand read cover meet in distinct positions
+// (head_dim 64: 8 chunks a row of 128 bytes, swizzled as the Vt rows below)
+template <int D>
+__device__ __forceinline__ int fa_kpos(int r, int c) {
+    return D == 128 ? c ^ (fa_swap23(r) & 15) : c ^ ((r >> 1) & 7);
+}
+template <int D>
 __device__ __forceinline__ uint32_t fa_kswz(int r, int c) {
-    return (uint32_t)(r * 256 + ((c ^ (fa_swap23(r) & 15)) << 4));
+    return (uint32_t)(r * (D * 2) + (fa_kpos<D>(r, c) << 4));
 }
 // byte offset of 16-byte chunk c (8 keys) of Vt tile row d (8 chunks a row),
 // XOR-swizzled by d / 2 % 8.  A 16-byte read is served 16 lanes (256 bytes, every
@@ -88,13 +106,21 @@ __device__ __forceinline__ uint32_t fa_kswz(int r, int c) {
 // rows d and d + 8 on the same banks: 4 conflict cycles a read, measured)
 __device__ __forceinline__ uint32_t fa_vswz(int d, int c) { return (uint32_t)(d * 128 + ((c ^ ((d >> 1) & 7)) << 4)); }
 
+// s + lo + hi of a bf16 pair
+__device__ __forceinline__ float fa_add_pair(uint32_t pair, float s) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_vt, pair), __builtin_bit_cast(bf16x2_vt, 0x3F803F80u),
+                                           s, false);
+}
+
 // ADD: the additive mask (attention.py:449-450).  Every block adds the column's mask
 // row (finite values clamped to -FLT_MAX in the kernel's units, -inf kept), loaded one
 // block ahead into registers; a column's running maximum may then stay -inf for whole
 // blocks, so probabilities of -inf scores are set to 0 explicitly, and a column whose
 // every visible score is -inf ends as 0 / 0 = NaN, as the reference's softmax does.
-template <bool ADD>
-__global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
+template <int D, bool ADD>
+__global__ void __launch_bounds__(FA_THREADS) __attribute__((amdgpu_waves_per_eu(D == 64 && !ADD ? 3 : 1)))
+attn_prefill_kernel(FaArgs a) {
+    using Gm = FaGeo<D>;
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int li = lane & 31, lh = lane >> 5;
@@ -126,19 +152,19 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
     // at or below need no mask
     const int wlimit = off + min(qb * PB + 32 * w / a.R, last_pos);
 
-    bf16x8_t qv[8];
+    bf16x8_t qv[Gm::KSTEPS];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
+    for (int ks = 0; ks < Gm::KSTEPS; ++ks) {
         uint4 v = make_uint4(0u, 0u, 0u, 0u);
         if (col_ok)
-            v = *reinterpret_cast<const uint4 *>(a.q + ((size_t)b * a.S + pos) * a.q_stride + (size_t)h * FA_D + 16 * ks + 8 * lh);
+            v = *reinterpret_cast<const uint4 *>(a.q + ((size_t)b * a.S + pos) * a.q_stride + (size_t)h * D + 16 * ks + 8 * lh);
         qv[ks] = as_bf16x8(v);
     }
     const int kend = off + last_pos + 1;               // keys [0, kend) are needed
     const int nblk = (kend + FA_KB - 1) / FA_KB;
     const int nfull = min(nblk, (wlimit + 1) / FA_KB);  // blocks with every key <= wlimit
-    const uint16_t *kbase = a.kc + ((size_t)b * a.Hkv + hk) * (size_t)a.T_cap * FA_D;
-    const uint16_t *vbase = a.vt + ((size_t)b * a.Hkv + hk) * (size_t)FA_D * a.T_cap;
+    const uint16_t *kbase = a.kc + ((size_t)b * a.Hkv + hk) * (size_t)a.T_cap * D;
+    const uint16_t *vbase = a.vt + ((size_t)b * a.Hkv + hk) * (size_t)D * a.T_cap;
 
     // staging of a block, all by LDS-DMA (no registers; explicit vmcnt waits, the
     // only vector-memory operations of the loop): wave w issues K instructions
@@ -147,19 +173,20 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
     // position i % 8), each lane loading the chunk the swizzle puts at its position.
     // Blocks are issued one ahead into a 2-stage ring.
     auto stage_blk = [&](int kb, int st) {
-        const uint32_t kl = (uint32_t)(uintptr_t)(smem + st * FA_STAGE);
-        const uint32_t vl = kl + FA_KTILE;
+        const uint32_t kl = (uint32_t)(uintptr_t)(smem + st * Gm::STAGE);
+        const uint32_t vl = kl + Gm::KTILE;
 #pragma unroll
-        for (int qq = 0; qq < 4; ++qq) {
-            const int qi = 4 * w + qq;
-            const int r = 4 * qi + (lane >> 4);
-            const int c = (lane & 15) ^ (fa_swap23(r) & 15);
+        for (int qq = 0; qq < Gm::DMA; ++qq) {
+            const int qi = Gm::DMA * w + qq;
+            constexpr int CPR = Gm::KROW / 16;             // chunks of a key row
+            const int r = Gm::KROWS_PI * qi + lane / CPR;
+            const int c = fa_kpos<D>(r, lane % CPR);
             const int key = min(kb + r, a.T_cap - 1);
-            dma::dma16s(kbase, (uint32_t)(key * (FA_D * 2) + 16 * c), kl + 1024 * qi);
+            dma::dma16s(kbase, (uint32_t)(key * Gm::KROW + 16 * c), kl + 1024 * qi);
         }
 #pragma unroll
-        for (int qq = 0; qq < 4; ++qq) {
-            const int qi = 4 * w + qq;
+        for (int qq = 0; qq < Gm::DMA; ++qq) {
+            const int qi = Gm::DMA * w + qq;
             const int d = 8 * qi + (lane >> 3);
             const int c = (lane & 7) ^ ((d >> 1) & 7);
             // T_cap is a multiple of 32, so only chunks wholly past the capacity clamp
@@ -168,9 +195,9 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
         }
     };
 
-    f32x16_t o[4];
+    f32x16_t o[Gm::DB];
 #pragma unroll
-    for (int db = 0; db < 4; ++db) o[db] = f32x16_t{};
+    for (int db = 0; db < Gm::DB; ++db) o[db] = f32x16_t{};
     float m = -INFINITY, lsum = 0.f;
 
     // the column's mask row and the 32 values of the next block (register r of half kh:
@@ -199,7 +226,7 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
     // DMA, and a wait it placed at q's first use would sit in the loop and also wait
     // for the blocks in flight every iteration
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" ::"v"(qv[ks]));
+    for (int ks = 0; ks < Gm::KSTEPS; ++ks) asm volatile("" ::"v"(qv[ks]));
     dma::wait_vm<0>();
     __syncthreads();
     const float sc = a.scale_log2;
@@ -210,8 +237,8 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
         constexpr bool MASK = decltype(mask_tag)::value;
         constexpr int st = decltype(stage_tag)::value;
         const int kb = blk * FA_KB;
-        const uint8_t *K = smem + st * FA_STAGE;
-        const uint8_t *V = K + FA_KTILE;
+        const uint8_t *K = smem + st * Gm::STAGE;
+        const uint8_t *V = K + Gm::KTILE;
         // block blk + 1 goes to the stage block blk - 1 used (read before the last barrier)
         if (blk + 1 < nblk) stage_blk(kb + FA_KB, st ^ 1);
 
@@ -223,16 +250,16 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
         f32x16_t sacc[2] = {f32x16_t{}, f32x16_t{}};
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
+        for (int ks = 0; ks < Gm::KSTEPS; ++ks)
 #pragma unroll
             for (int kh = 0; kh < 2; ++kh) {
-                const bf16x8_t ka = as_bf16x8(*reinterpret_cast<const uint4 *>(K + fa_kswz(32 * kh + arow, 2 * ks + lh)));
+                const bf16x8_t ka = as_bf16x8(*reinterpret_cast<const uint4 *>(K + fa_kswz<D>(32 * kh + arow, 2 * ks + lh)));
                 sacc[kh] = mfma32x32x16(ka, qv[ks], sacc[kh]);
             }
 #pragma unroll
         for (int i = 0; i < FA_SAHEAD; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #pragma unroll
-        for (int i = 0; i < 16 - FA_SAHEAD; ++i) {
+        for (int i = 0; i < 2 * Gm::KSTEPS - FA_SAHEAD; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
@@ -268,12 +295,18 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
             for (int r = 0; r < 16; ++r) bm = fmaxf(bm, sacc[kh][r]);
         bm = fmaxf(bm, __shfl_xor(bm, 32));
         float alpha = 1.f;
-        if ((bm - m) * sc > 8.f) {
+        if ((bm - m) * sc > Gm::LAZY) {
             alpha = __builtin_amdgcn_exp2f((m - bm) * sc);
             m = bm;
         }
         const float nms = -m * sc;
+        // The probabilities in bf16, and the column's sum of those same rounded values: the
+        // roundings then cancel in O / l where few keys carry the weight (summed before the
+        // rounding, positions of few keys were up to 10 % further from the exact result),
+        // and v_dot2 adds a pair per instruction
         float ps = 0.f;
+        uint32_t pk[2][8];
+        float phold = 0.f;
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
@@ -288,14 +321,17 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
                 } else {
                     p = __builtin_amdgcn_exp2f(fmaf(sacc[kh][r], sc, nms));
                 }
-                sacc[kh][r] = p;
-                ps += p;
+                if (r & 1) {
+                    pk[kh][r >> 1] = cvt_pk_bf16(phold, p);
+                    ps = fa_add_pair(pk[kh][r >> 1], ps);
+                }
+                phold = p;
             }
         lsum = lsum * alpha + ps;
         // rescale O^T only when some column's maximum moved (wave-uniform test)
         if (__ballot(alpha != 1.f) != 0ull) {
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < Gm::DB; ++db)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
         }
@@ -305,11 +341,8 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
-            const int kh = s4 >> 1, r0 = 8 * (s4 & 1);
-            const bf16x8_t pb = as_bf16x8(cvt_pk_bf16(sacc[kh][r0], sacc[kh][r0 + 1]),
-                                          cvt_pk_bf16(sacc[kh][r0 + 2], sacc[kh][r0 + 3]),
-                                          cvt_pk_bf16(sacc[kh][r0 + 4], sacc[kh][r0 + 5]),
-                                          cvt_pk_bf16(sacc[kh][r0 + 6], sacc[kh][r0 + 7]));
+            const int kh = s4 >> 1, p0 = 4 * (s4 & 1);
+            const bf16x8_t pb = as_bf16x8(pk[kh][p0], pk[kh][p0 + 1], pk[kh][p0 + 2], pk[kh][p0 + 3]);
             const int c = 4 * kh + 2 * (s4 & 1) + lh;
             // cache slots at or past T may hold anything, NaN included: their zero
             // probabilities must not meet them, so the V pieces of the block that
@@ -323,7 +356,7 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
                 mk.w = (k0 + 6 < T ? 0xFFFFu : 0u) | (k0 + 7 < T ? 0xFFFF0000u : 0u);
             }
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
+            for (int db = 0; db < Gm::DB; ++db) {
                 const uint4 v = *reinterpret_cast<const uint4 *>(V + fa_vswz(32 * db + li, c));
                 o[db] = mfma32x32x16(as_bf16x8(v.x & mk.x, v.y & mk.y, v.z & mk.z, v.w & mk.w), pb, o[db]);
             }
@@ -331,7 +364,7 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
 #pragma unroll
         for (int i = 0; i < FA_SAHEAD; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #pragma unroll
-        for (int i = 0; i < 16 - FA_SAHEAD; ++i) {
+        for (int i = 0; i < 4 * Gm::DB - FA_SAHEAD; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
@@ -359,9 +392,9 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
     const float ltot = lsum + __shfl_xor(lsum, 32);
     if (!col_ok) return;
     const float inv = (ADD || ltot > 0.f) ? 1.f / ltot : 0.f;
-    uint16_t *orow = a.out + ((size_t)b * a.S + pos) * a.out_stride + (size_t)h * FA_D;
+    uint16_t *orow = a.out + ((size_t)b * a.S + pos) * a.out_stride + (size_t)h * D;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < Gm::DB; ++db)
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             const int d = 32 * db + 8 * r4 + 4 * lh;
@@ -373,7 +406,21 @@ __global__ void __launch_bounds__(FA_THREADS) attn_prefill_kernel(FaArgs a) {
 
 }  // namespace
 
-// Launches attn_prefill_kernel when the shape suits it (head_dim 128, the GQA ratio
+template <int D, bool ADD>
+static int launch_fa(const FaArgs &f, long wgs, hipStream_t stream) {
+    static bool configured = false;
+    auto kern = attn_prefill_kernel<D, ADD>;
+    if (!configured) {
+        SC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, FaGeo<D>::LDS));
+        configured = true;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(FA_THREADS), FaGeo<D>::LDS, stream, f);
+    SC_HIP_CHECK(hipGetLastError());
+    return SC_OK;
+}
+
+// Launches attn_prefill_kernel when the shape suits it (head_dim 128 or 64, the GQA ratio
 // dividing 128, 16-byte aligned Vt, at least 128 / R new positions: one workgroup's
 // columns) and returns SC_OK; returns 1, launching nothing, when it does not.  The
 // choice does not depend on the batch size, so that a sequence's result is the same
@@ -384,7 +431,15 @@ int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, co
                         const int32_t *cache_len, uint16_t *out, long out_stride, long B, long S, long H, long Hkv,
                         long D, float scale, hipStream_t stream, const float *mask, const long *ms) {
     const long R = H / Hkv;
-    if (D != FA_D || FA_COLS % R != 0 || ((uintptr_t)vt % 16) != 0) return 1;
+    if ((D != 128 && D != 64) || FA_COLS % R != 0 || ((uintptr_t)vt % 16) != 0) return 1;
+    // head_dim 64: few query rows over many keys stay on attn_kernel, which splits the keys
+    // over workgroups (a workgroup here takes ~1 us per 64 keys).  Measured, one sequence,
+    // 32 q heads on 4 kv heads, attn_kernel -> here: 128 positions after 1500 16 -> 26 us,
+    // 192 24 -> 27, 256 25 -> 28, 384 47 -> 29; 384 after 300 26 -> 14, 64 after 300
+    // 14 -> 11; 8 heads of their own: 1024 after 1500 34 -> 38, 1024 after 300 25 -> 23; 701
+    // positions of 3 sequences 84 -> 19, 2048 of one 163 -> 37.  By the capacity and not
+    // the length, which only the device knows.
+    if (D == 64 && S * H < 12288 && T_cap > 512) return 1;
     if (T_cap > (1L << 22)) return 1;    // staging offsets within one (b, kv head) slab are 32-bit
     const long nqb = (S + FA_COLS / R - 1) / (FA_COLS / R);
     const long wgs = B * Hkv * nqb;
@@ -399,17 +454,9 @@ int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, co
     f.mask = mask;
     f.msb = mask ? ms[0] : 0; f.msh = mask ? ms[1] : 0; f.mss = mask ? ms[2] : 0; f.mst = mask ? ms[3] : 0;
     f.mask_unscale = 1.f / scale;
-    static bool configured[2] = {false, false};
-    if (!configured[mask != nullptr]) {
-        SC_HIP_CHECK(hipFuncSetAttribute(mask ? reinterpret_cast<const void *>(attn_prefill_kernel<true>)
-                                              : reinterpret_cast<const void *>(attn_prefill_kernel<false>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS));
-        configured[mask != nullptr] = true;
-    }
-    if (mask) hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3((unsigned)wgs), dim3(FA_THREADS), FA_LDS, stream, f);
-    else hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3((unsigned)wgs), dim3(FA_THREADS), FA_LDS, stream, f);
-    SC_HIP_CHECK(hipGetLastError());
-    return SC_OK;
+    if (D == 128)
+        return mask ? launch_fa<128, true>(f, wgs, stream) : launch_fa<128, false>(f, wgs, stream);
+    return mask ? launch_fa<64, true>(f, wgs, stream) : launch_fa<64, false>(f, wgs, stream);
 }
 
 }  // namespace sc

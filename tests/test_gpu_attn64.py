@@ -1,0 +1,65 @@
+"""Prefill attention at head_dim 64 on the 128-column kernel against float64: positions at the
+edges of a workgroup's columns (128 / R positions), GQA ratios 8, 4 and 1, cached prefixes,
+garbage past the length, an additive mask, and both sides of the rule that keeps few query
+rows over a large cache on the key-splitting kernel.
+
+The bound is the attention's: bf16 probabilities and outputs, max |y - ref| <= 1e-2 max |ref|."""
+import math
+
+import pytest
+import torch
+
+from shardcompute_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+D = 64
+
+
+def _reference(q, k, v, past, mask):
+    """q [B, H, S, D], k and v [B, Hkv, T, D] in float64."""
+    B, H, S, _ = q.shape
+    T, R = k.shape[2], H // k.shape[1]
+    hidden = torch.arange(T, device=q.device)[None] > torch.arange(past, past + S, device=q.device)[:, None]
+    out = torch.empty_like(q)
+    for b in range(B):
+        for h in range(H):
+            s = q[b, h] @ k[b, h // R].T.contiguous() / math.sqrt(D)
+            if mask is not None:
+                s = s + mask[b].double()
+            out[b, h] = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[b, h // R]
+    return out
+
+
+# (B, S, H, Hkv, past, T_cap): the last two on either side of S H = 12288 with a large cache
+CASES = [(1, 16, 32, 4, 0, 32), (2, 17, 32, 4, 47, 96), (1, 33, 16, 4, 0, 64), (2, 129, 4, 4, 5, 160),
+         (1, 100, 8, 1, 300, 512), (3, 200, 32, 4, 0, 224), (1, 383, 32, 4, 400, 1024), (1, 385, 32, 4, 400, 1024)]
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,past,T_cap", CASES)
+@pytest.mark.parametrize("masked", [False, True])
+def test_prefill_attention_head_dim_64(device, B, S, H, Hkv, past, T_cap, masked):
+    print(f"attention64 B={B} S={S} H={H} Hkv={Hkv} past={past} T_cap={T_cap} masked={masked}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(S + past)
+    T = past + S
+    q = torch.randn((B * S, H * D), generator=g, device="cuda").to(torch.bfloat16)
+    kc = torch.randn((B, Hkv, T_cap, D), generator=g, device="cuda").to(torch.bfloat16)
+    vt = torch.randn((B, Hkv, D, T_cap), generator=g, device="cuda").to(torch.bfloat16)
+    mask = None
+    if masked:
+        # left padding of the first key of odd rows and a random bias elsewhere
+        mask = torch.randn((B, 1, 1, T), generator=g, device="cuda")
+        if T > 1:
+            mask[1::2, :, :, :1] = torch.finfo(torch.float32).min
+    kd, vd = kc[:, :, :T].double(), vt[:, :, :, :T].double().transpose(2, 3).contiguous()
+    kc[:, :, T:] = float("nan")
+    vt[:, :, :, T:] = float("nan")
+    cnt = torch.tensor([past, 0], dtype=torch.int32, device="cuda")
+    out = _lib.attention(q, B, S, H, Hkv, D, kc, vt, cnt, 1 / math.sqrt(D), mask=mask, n_keys=T)
+    torch.cuda.synchronize()
+    ref = _reference(q.view(B, S, H, D).transpose(1, 2).double(), kd, vd, past,
+                     None if mask is None else mask[:, 0])
+    got = out.view(B, S, H, D).transpose(1, 2).double()
+    assert torch.isfinite(got).all()
+    assert (got - ref).abs().max() <= 1e-2 * ref.abs().max()

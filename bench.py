@@ -535,11 +535,15 @@ def bench_lm_head_m64(reps=10):
             "frac_hbm": round(gbs / HBM_PEAK_GBS, 4), "TFLOPs": round(tf, 1)}
 
 
-def qmm_kernel_label(M, N, K, cus=256):
-    """The kernel sc_qmm_bf16's automatic path takes for an M x K -> N product (the
-    choice csrc/abi.hip and csrc/qgemm.hip make, restated for the sweep's labels)."""
+def qmm_kernel_label(M, N, K, bits, cus=256):
+    """The kernel the automatic path takes for an M x K -> N product (the choice
+    csrc/abi.hip, csrc/qgemm_dense.hip and csrc/qgemm.hip make, restated for the sweep's
+    labels)."""
+    from shardcompute_amd import _lib
+    if _lib.load().sc_qmm_workspace_bytes(M, N, K) > 0:
+        return "dequantize + dense gemm"
     band = K % 512 == 0 and (M <= 160 if M > 32 else K >= 4096 if M == 8 else
-                             M > 8 and (K > 4096 or N <= 8192))
+                             M > 16 or M > 8 and (K > 4096 or N <= (16384 if bits == 4 else 65536)))
     if band:
         return "band"
     if M <= 32:
@@ -605,7 +609,7 @@ def bench_qmm_sweep(reps=5):
                 us = e0.elapsed_time(e1) * 1e3 / (reps * copies)
                 nbytes = qmm_bytes(M, N, K, bits)
                 flops = 2.0 * M * N * K
-                kernel = qmm_kernel_label(M, N, K)
+                kernel = qmm_kernel_label(M, N, K, bits)
                 row = {"bits": bits, "M": M, "K": K, "N": N, "kernel": kernel, "gpu_us": round(us, 2)}
                 if M <= 32:
                     gbs = nbytes / (us * 1e-6) / 1e9

@@ -170,15 +170,19 @@ static int check_qmm(const void *x, const void *wq, const void *s, const void *b
 // kernels compute 32 rows and the band's stream is the faster (8B gate|up at 20, 24
 // and 32 rows 28, 31, 30 against 32, 34, 34 us on the GEMV; the 8B lm_head at 32 rows
 // 99 against 119 us); 9-16 rows where the 16-column GEMV's K splits or x staging cost
-// more than the band's stream: K above 4096 or at most 8192 weight rows (8B down at 16
-// rows 17 against 25 us; 8B gate|up at 16 rows 29 against 24 us and the lm_head 95
-// against 73 us stay on the GEMV, which computes 16 rows where the band computes 32);
-// and 8 rows with K of 4096 or more (8B q|k|v, gate|up, down 10, 15, 16 against 12,
-// 17, 26 us on the 8-row GEMV; K = 2048 is a tie).
-static bool band_first(int64_t M, int64_t N, int64_t K) {
+// more than the band's stream: K above 4096, or up to 16384 weight rows at 4 bits and
+// 65536 at 8 (TinyLlama gate|up at 16 rows 11.5 against 12.0 us, W8 12.2 against 15.0; 8B
+// gate|up W8 34.0 against 38.5, W4 24.6 against 24.4; the 8B lm_head 77 against 70, W8 139
+// against 135);
+// and 8 rows with K of 4096 or more (8B q|k|v, gate|up, down 10, 24, 16 against 13,
+// 25, 26 us on the 8-row GEMV; K = 2048 is a tie).  4-7 rows, and 8 rows of a smaller K, are
+// up to 1.6 times faster here too (8B down at 4 rows 16 against 25 us), but stay on the GEMV:
+// it needs no split-K scratch, so those products may run on several streams at once and
+// be a process's first call under capture.
+static bool band_first(int64_t M, int64_t N, int64_t K, int bits) {
     if (M > 32) return M <= 160;
     if (M == 8) return K >= 4096;
-    return M > 16 || (M > 8 && (K > 4096 || N <= 8192));
+    return M > 16 || (M > 8 && (K > 4096 || N <= (bits == 4 ? 16384 : 65536)));
 }
 
 // The caller's workspace of a call (none: ws null), for the products whose weights are
@@ -199,7 +203,7 @@ static int qmm_dispatch(const uint16_t *x, const uint32_t *wq, const uint16_t *s
         rc = launch_qgemm_dense(x, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, 0, wsp.ws, wsp.bytes);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
-    if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
+    if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K, bits) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
                                                                                     : SC_QMM_PATH_GEMM;
     if (path == SC_QMM_PATH_BAND) {
         // any M <= 256: the weight-streaming band kernel; shapes it does not take (K not
@@ -301,7 +305,7 @@ static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw,
                                 wsp.bytes);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
-    if (band_first(M, N, K)) {
+    if (band_first(M, N, K, bits)) {
         // the band kernel's split-K pass applies silu(gate) * up itself
         rc = launch_qgemm_band(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half, 0,
                                0);

@@ -106,12 +106,6 @@ __device__ __forceinline__ uint32_t fa_kswz(int r, int c) {
 // rows d and d + 8 on the same banks: 4 conflict cycles a read, measured)
 __device__ __forceinline__ uint32_t fa_vswz(int d, int c) { return (uint32_t)(d * 128 + ((c ^ ((d >> 1) & 7)) << 4)); }
 
-// s + lo + hi of a bf16 pair
-__device__ __forceinline__ float fa_add_pair(uint32_t pair, float s) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_vt, pair), __builtin_bit_cast(bf16x2_vt, 0x3F803F80u),
-                                           s, false);
-}
-
 // ADD: the additive mask (attention.py:449-450).  Every block adds the column's mask
 // row (finite values clamped to -FLT_MAX in the kernel's units, -inf kept), loaded one
 // block ahead into registers; a column's running maximum may then stay -inf for whole
@@ -323,7 +317,7 @@ attn_prefill_kernel(FaArgs a) {
                 }
                 if (r & 1) {
                     pk[kh][r >> 1] = cvt_pk_bf16(phold, p);
-                    ps = fa_add_pair(pk[kh][r >> 1], ps);
+                    ps = add_pair_bf16(pk[kh][r >> 1], ps);
                 }
                 phold = p;
             }

@@ -1,4 +1,4 @@
-// Kernel C: the middle band of the quantized product, 9 <= M <= 256 rows of x.
+// Kernel C: the middle band of the quantized product, 8 <= M <= 256 rows of x.
 //
 // y[m, n] = sum_k x[m, k] * (s[n, k/64] * q[n, k] + b[n, k/64])
 // (mx.quantized_matmul(x, wq, s, b, transpose=True, group_size=64, bits),
@@ -41,7 +41,11 @@
 //   with several, each split writes fp32 partials and the split-K pass sums them in
 //   split order (deterministic).
 #include "dma_util.h"
+
 #include "../../include/shardcompute_hip.h"
+
+#include <type_traits>
+#include <utility>
 
 namespace sc {
 
@@ -62,30 +66,48 @@ namespace band {
 using namespace dma;
 
 constexpr int NP = 4;                                  // producer waves
-constexpr int LDS_CAP = 152 * 1024;
+constexpr int LDS_CAP = 160 * 1024;
 
-// x ring slots that fit beside the code and scale/bias rings, capped where the code
-// ring's refill would overtake its readers (x runs NX - 1 stages ahead; a code item is
-// loaded over the IG stages before its first use, into the slot two items back:
-// NX - 1 < IG + 2)
-__host__ __device__ constexpr int band_nx(int bits, int mt, int nw) {
-    return ((LDS_CAP - 3 * (32 * nw * 128) - 2 * (1024 * nw)) / (mt * 4096)) < (bits == 4 ? 6 : 4)
-               ? ((LDS_CAP - 3 * (32 * nw * 128) - 2 * (1024 * nw)) / (mt * 4096))
-               : (bits == 4 ? 6 : 4);
+// bytes of an x stage: 32 mt rows (mt = 0: 16 rows) of 64 bf16
+__host__ __device__ constexpr int band_xb(int mt) { return mt == 0 ? 2048 : mt * 4096; }
+// The rings' slots: nx x stages and ns code items.  The stream's rate is the bytes in
+// flight, nx - 2 stages' lists, so the pair with the most x slots that fits is taken:
+// * the code ring's refill must not overtake its readers (x runs lx = nx - 1 stages ahead;
+//   an item is loaded over the ig stages of the item before it): lx <= ig (ns - 2) + 1;
+// * a scale/bias block's refill must not overtake its one read: lx <= 7;
+// * 4-wave workgroups of up to 32 rows stay within half the LDS, two to a CU;
+// * W8 above 32 rows keeps 3 code items: with 5 (two to three times the bytes in flight)
+//   its first stage starts later and a 45-row product of any size took 1.3 us longer.
+// 4 items where 3 were: 45 rows W4, 4096 -> 6144 16.3 -> 14.9 us, 14336 -> 4096 22.4 -> 19.4.
+struct Rings {
+    int nx, ns;
+};
+__host__ __device__ constexpr Rings band_rings(int bits, int mt, int nw) {
+    const int cap = mt <= 1 && nw == 4 ? 80 * 1024 : LDS_CAP;
+    const int ig = bits == 4 ? 4 : 2, item = 32 * nw * 128;
+    Rings best{0, 3};
+    for (int ns = 3; ns <= (bits == 8 && mt >= 2 ? 3 : 6); ++ns) {
+        int nx = (cap - ns * item - 2 * (1024 * nw)) / band_xb(mt);
+        if (nx > ig * (ns - 2) + 2) nx = ig * (ns - 2) + 2;
+        if (nx > 8) nx = 8;
+        if (nx > best.nx) best = Rings{nx, ns};
+    }
+    return best;
 }
 
 template <int BITS, int MT, int NW>
 struct Geo {
     static constexpr int BN = 32 * NW;                 // weight rows per workgroup
-    static constexpr int XB = MT * 32 * 128;           // x stage: 32 MT rows x 64 bf16
+    static constexpr int XB = band_xb(MT);             // x stage: 32 MT (or 16) rows x 64 bf16
     static constexpr int WROW = BITS == 4 ? 32 : 64;   // bytes of one weight row per group
     static constexpr int IG = 128 / WROW;              // groups per code item
     static constexpr int WIB = BN * 128;               // code item bytes
     static constexpr int SBB = 2 * BN * 16;            // scales then biases, 8 groups of BN rows
-    static constexpr int NX = band_nx(BITS, MT, NW);   // x ring slots
+    static constexpr int NX = band_rings(BITS, MT, NW).nx;   // x ring slots
+    static constexpr int NS = band_rings(BITS, MT, NW).ns;   // code ring slots
     static constexpr int LX = NX - 1;                  // stages the x DMA runs ahead
     static constexpr int O_W = NX * XB;                // LDS: x ring, code ring, s/b slots
-    static constexpr int O_SB = O_W + 3 * WIB;
+    static constexpr int O_SB = O_W + NS * WIB;
     static constexpr int LDS = O_SB + 2 * SBB;
     static constexpr int XI = XB / 1024;               // DMA instructions per stage: x,
     static constexpr int WPI = WIB / 1024 / IG;        // a piece of a code item,
@@ -93,14 +115,148 @@ struct Geo {
     static constexpr int DP = (TI + NP - 1) / NP;      // per producer: DP or DP - 1
     static constexpr int NFULL = TI % NP == 0 ? NP : TI % NP;   // producers issuing DP
     static constexpr int THREADS = 64 * (NW + NP);
-    static_assert(NX >= 2 && LX < IG + 2, "x ring");
+    static_assert(NX >= 3 && LX <= IG * (NS - 2) + 1 && LX <= 7, "rings");
     static_assert(LDS <= LDS_CAP, "LDS");
     static_assert((LX - 1) * DP < 64, "vmcnt range");
 };
 
+// stage(number of lists issued after it, false, its index) for the last sizeof...(Is) stages
+template <class F, int... Is>
+__device__ __forceinline__ void tail_stages(F &&stage, int g, std::integer_sequence<int, Is...>) {
+    constexpr int L = (int)sizeof...(Is);
+    (stage(std::integral_constant<int, L - 1 - Is>{}, false, g + Is), ...);
+}
+
 }  // namespace band
 
 using namespace band;
+
+// Up to 16 rows (MT = 0): the consumers' loop, by the rule of the 17-32-row one below (exact
+// codes on MFMA, y += s P + (b - 128 s) S in fp32) at half its work:
+// * 16x16x32 MFMAs on two blocks of 16 weight rows: half the MFMA time, x operands and
+//   scale FMAs of a 32-row block;
+// * (b - 128 s) S is one fp32 MFMA per block and group: A holds each lane's own part of the
+//   row's x sum (v_dot2 with ones over the operands it has), B the column's b - 128 s in
+//   every k slot, so the contraction adds the parts up, instead of a second bf16 MFMA
+//   chain with all-ones weights and 4 more FMAs.  (Summing a group's x in one wave and
+//   sharing it through LDS is less work still, but as a branch of the unrolled stages it
+//   doubled the registers.)
+// Measured with its split-K pass, this and the shorter tail of the stream (us, 16 rows,
+// before -> after): W4 4096 -> 6144 11.9 -> 10.8, 14336 -> 4096 17.5 -> 16.3, 8192 -> 7168
+// 17.8 -> 16.0, 3584 -> 8192 12.4 -> 11.3; W8 12.8 -> 12.3, 20.6 -> 19.9, 19.8 -> 19.6, 14.1 -> 13.7.
+template <int BITS, int NW>
+__device__ __forceinline__ void consume16(const BandArgs &a, uint8_t *smem, int wave, int lane, int n0, int nb,
+                                          int split) {
+    using C = Geo<BITS, 0, NW>;
+    constexpr int NX = C::NX, IG = C::IG;
+    const int li = lane & 15, lq = lane >> 4;          // operand row (column), k part
+    uint32_t nib16 = 0x000F000Fu, magic = 0x43004300u; // opaque: one v_and_or_b32 per code pair
+    asm volatile("" : "+s"(nib16));
+    asm volatile("" : "+v"(magic));
+    f32x4_t acc[2] = {f32x4_t{}, f32x4_t{}};
+    // lane part lq's k-step ks takes k chunk 2 lq + ks of the group (8 k), for x and codes
+    // alike, so that a lane's codes of the group are contiguous
+    uint32_t xo[2], wo[2];
+    int wsw[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+        xo[ks] = (uint32_t)(li * 128 + (((2 * lq + ks) ^ (li & 7) ^ ((li >> 3) & 1)) << 4));
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int rr = 32 * wave + 16 * c + li;
+        wo[c] = (uint32_t)(C::O_W + rr * 128);
+        wsw[c] = (rr >> 1) & 7;
+    }
+    uint4 sv[2], bv[2];                                // scales, biases of the block's 8 groups
+    int xslot = 0, wslot = 0;
+    for (int bk = 0; bk < nb; ++bk) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __syncthreads();                           // stage 8 bk + j landed
+            if (j == 0) {
+                const uint8_t *sb = smem + C::O_SB + (bk & 1) * C::SBB;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    sv[c] = *reinterpret_cast<const uint4 *>(sb + 16 * (32 * wave + 16 * c + li));
+                    bv[c] = *reinterpret_cast<const uint4 *>(sb + 16 * (C::BN + 32 * wave + 16 * c + li));
+                }
+            }
+            const uint8_t *xs = smem + xslot * C::XB;
+            const uint8_t *ws = smem + wslot * C::WIB;
+            const int gi = j % IG;                     // group of the code item
+            uint4 xv[2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) xv[ks] = *reinterpret_cast<const uint4 *>(xs + xo[ks]);
+            uint32_t w[2][BITS == 4 ? 2 : 4];          // the lane's codes of the group
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if constexpr (BITS == 4) {
+                    const uint2 v = *reinterpret_cast<const uint2 *>(
+                        ws + wo[c] + ((((2 * gi + (lq >> 1)) ^ wsw[c]) << 4) | ((lq & 1) << 3)));
+                    w[c][0] = v.x; w[c][1] = v.y;
+                } else {
+                    const uint4 v = *reinterpret_cast<const uint4 *>(ws + wo[c] + (((4 * gi + lq) ^ wsw[c]) << 4));
+                    w[c][0] = v.x; w[c][1] = v.y; w[c][2] = v.z; w[c][3] = v.w;
+                }
+            }
+            f32x4_t P[2] = {f32x4_t{}, f32x4_t{}};
+            float sx = 0.f;                            // this lane's part of the group's x sum
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                sx = add_pair_bf16(xv[ks].x, sx);
+                sx = add_pair_bf16(xv[ks].y, sx);
+                sx = add_pair_bf16(xv[ks].z, sx);
+                sx = add_pair_bf16(xv[ks].w, sx);
+                const bf16x8_t A = as_bf16x8(BITS == 4 ? perm_w4x(xv[ks]) : xv[ks]);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    bf16x8_t B;
+                    if constexpr (BITS == 4) {
+                        const uint32_t v = w[c][ks];
+                        B = as_bf16x8(and_or(v, nib16, magic), and_or(v >> 4, nib16, magic),
+                                      and_or(v >> 8, nib16, magic), and_or(v >> 12, nib16, magic));
+                    } else {
+                        const uint32_t w0 = w[c][2 * ks], w1 = w[c][2 * ks + 1];
+                        B = as_bf16x8(byte_pair_lo(w0), byte_pair_hi(w0), byte_pair_lo(w1), byte_pair_hi(w1));
+                    }
+                    P[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, P[c], 0, 0, 0);
+                }
+            }
+            // the compiler leaves no wait states between a v_dot2 and the MFMA that reads its
+            // result (the last terms of the sum were missing): 4 here
+            asm volatile("s_nop 3" : "+v"(sx));
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float sf = bf2f(wh(sv[c], j)), bf = bf2f(wh(bv[c], j));
+                acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, BITS == 4 ? fmaf(-128.f, sf, bf) : bf, acc[c], 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[c][r] = fmaf(sf, P[c][r], acc[c][r]);
+            }
+            xslot = xslot + 1 == NX ? 0 : xslot + 1;
+            if (j % IG == IG - 1) wslot = wslot + 1 == C::NS ? 0 : wslot + 1;
+        }
+    }
+
+    // lane (column li, part lq) register r holds row 4 lq + r
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int n = n0 + 32 * wave + 16 * c + li;
+        if (n >= a.N) continue;
+        const float bb = (!a.partials && a.bias) ? bf2f(a.bias[n]) : 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = 4 * lq + r;
+            if (m >= a.M) continue;
+            if (a.partials) {
+                a.partials[((size_t)split * a.M + m) * a.N + n] = acc[c][r];
+            } else {
+                uint32_t o = f2bf(acc[c][r]);
+                if (a.bias) o = f2bf(bf2f(o) + bb);
+                a.y[(size_t)m * a.N + n] = (uint16_t)o;
+            }
+        }
+    }
+}
 
 // The LDS holds one workgroup per CU, so (NW + NP) / 4 waves share a SIMD.  With 8 x
 // blocks the compiler, left to aim for more waves, keeps the accumulators and x
@@ -132,9 +288,9 @@ qgemm_band_kernel(BandArgs a) {
         // last piece rides with stage IG j, so waiting for stage IG j's x covers it),
         // the scale/bias instruction t % 8 of block t / 8 + 1 (repeats of the last
         // instruction when the block has fewer than 8; block b's last rides with stage
-        // 8b - 1), then the x stage.  Instruction i goes to producer i % NP.  Indices
-        // past the split are clamped: the reloads rewrite slots nobody reads any more
-        // (or the same bytes).
+        // 8b - 1), then the x stage.  Instruction i goes to producer i % NP.  Items,
+        // blocks and stages past the split are clamped: the reloads rewrite slots nobody reads any
+        // more (or the same bytes), and keep the lists' lengths equal.
         const int pw = wave - NW;
         const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
         const uint8_t *xbase = reinterpret_cast<const uint8_t *>(a.x) + (size_t)g0 * 128;
@@ -164,7 +320,7 @@ qgemm_band_kernel(BandArgs a) {
         auto issue_w = [&](int item, int q) __attribute__((always_inline)) {
             // instruction q of code item `item` (clamped to the split) into its slot
             const int ic = min(item, ni - 1);
-            dma16s(wbase + (size_t)ic * 128, woff(q), lds0 + C::O_W + (item % 3) * C::WIB + 1024 * q);
+            dma16s(wbase + (size_t)ic * 128, woff(q), lds0 + C::O_W + (item % C::NS) * C::WIB + 1024 * q);
         };
         auto issue = [&](int t) __attribute__((always_inline)) {
             const int tc = min(t, ng - 1);
@@ -183,13 +339,23 @@ qgemm_band_kernel(BandArgs a) {
         for (int q = pw; q < (IG - 1) * C::WPI; q += NP) issue_w(0, q);
         for (int u = pw; u < NW; u += NP) issue_sb(u, 0);
         for (int t = 0; t < LX; ++t) issue(t);
-        for (int g = 0; g < ng; ++g) {
-            // this producer's part of stage g (and everything it issued before) landed
-            if (pw < C::NFULL) wait_vm<(LX - 1) * C::DP>();
-            else wait_vm<(LX - 1) * (C::DP - 1)>();
+        auto stage = [&](auto after, bool more, int g) __attribute__((always_inline)) {
+            // this producer's part of stage g (and everything it issued before) landed; `after`
+            // lists were issued since
+            constexpr int n = decltype(after)::value;
+            if (pw < C::NFULL) wait_vm<n * C::DP>();
+            else wait_vm<n * (C::DP - 1)>();
             __syncthreads();                                // stage g visible; slots of g - 1 free
-            issue(g + LX);
-        }
+            if (more) issue(g + LX);
+        };
+        // The last LX stages (ng >= 8 > LX) have nothing left to issue: reloads of the last
+        // stage in their place (up to half a split's bytes again) cost 3-8 % of a product.
+        // Not so for W8 above 32 rows, where the two loops are 0.6 % slower than the reloads
+        // of its three lists (45 x 8192 -> 7168: 21.7 against 21.8 us).
+        constexpr bool TAIL = BITS == 4 || MT <= 1;
+        int g = 0;
+        for (; g < (TAIL ? ng - LX : ng); ++g) stage(std::integral_constant<int, LX - 1>{}, true, g);
+        if constexpr (TAIL) tail_stages(stage, g, std::make_integer_sequence<int, LX>{});
         wait_vm<0>();                                       // no DMA may land after the workgroup ends
         return;
     }
@@ -197,15 +363,19 @@ qgemm_band_kernel(BandArgs a) {
     // ==================================================================== consumers
     const int li = lane & 31, h = lane >> 5;
     const int rr = 32 * wave + li;                     // this lane's weight row in the tile
+    if constexpr (MT == 0) {
+        consume16<BITS, NW>(a, smem, wave, lane, n0, nb, split);
+        return;
+    }
     uint32_t nib = 0x0F0F0F0Fu;                        // opaque: one v_cvt_f32_ubyteN per code
     asm volatile("" : "+s"(nib));
     uint32_t nib16 = 0x000F000Fu, magic = 0x43004300u; // opaque: one v_and_or_b32 per code pair
     asm volatile("" : "+s"(nib16));
     asm volatile("" : "+v"(magic));
-    f32x16_t acc[MT];
+    constexpr int MB = MT > 1 ? MT : 1;
+    f32x16_t acc[MB];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) acc[i] = f32x16_t{};
-
+    for (int i = 0; i < MB; ++i) acc[i] = f32x16_t{};
     // x operand (row 32 i + li, 16-byte chunk 4 h + ks) of a stage
     auto xoff = [&](int i, int ks) -> uint32_t {
         const int r = 32 * i + li;
@@ -258,14 +428,14 @@ qgemm_band_kernel(BandArgs a) {
             return;
         }
         // x operands one k-step ahead of the MFMAs that use them
-        uint4 xa[2][MT];
+        uint4 xa[2][MB];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) xa[0][i] = *reinterpret_cast<const uint4 *>(xs + xoff(i, 0));
+        for (int i = 0; i < MB; ++i) xa[0][i] = *reinterpret_cast<const uint4 *>(xs + xoff(i, 0));
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             if (ks + 1 < 4) {
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
+                for (int i = 0; i < MB; ++i)
                     xa[(ks + 1) & 1][i] = *reinterpret_cast<const uint4 *>(xs + xoff(i, ks + 1));
             }
             bf16x8_t B;
@@ -285,7 +455,7 @@ qgemm_band_kernel(BandArgs a) {
                               cvt_pk_bf16(fmaf(sf, ubyte_f32(w1, 2), bf), fmaf(sf, ubyte_f32(w1, 3), bf)));
             }
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i] = mfma32x32x16(as_bf16x8(xa[ks & 1][i]), B, acc[i]);
+            for (int i = 0; i < MB; ++i) acc[i] = mfma32x32x16(as_bf16x8(xa[ks & 1][i]), B, acc[i]);
         }
     };
 
@@ -302,7 +472,7 @@ qgemm_band_kernel(BandArgs a) {
             }
             compute(xslot, wslot, j % IG, j, sv, bv);
             xslot = xslot + 1 == NX ? 0 : xslot + 1;
-            if (j % IG == IG - 1) wslot = wslot + 1 == 3 ? 0 : wslot + 1;
+            if (j % IG == IG - 1) wslot = wslot + 1 == C::NS ? 0 : wslot + 1;
         }
     }
 
@@ -312,7 +482,7 @@ qgemm_band_kernel(BandArgs a) {
     if (n < N) {
         const float bb = (!a.partials && a.bias) ? bf2f(a.bias[n]) : 0.f;
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
+        for (int i = 0; i < MB; ++i) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -360,7 +530,8 @@ static int launch_band_mt(const BandArgs &a, int nw, int tiles, int ksplit, hipS
 
 // LDS bytes of a variant (Geo<>::LDS)
 static int band_lds(int bits, int mt, int nw) {
-    return band_nx(bits, mt, nw) * mt * 4096 + 3 * (32 * nw * 128) + 2 * (1024 * nw);
+    const Rings r = band_rings(bits, mt, nw);
+    return r.nx * band_xb(mt) + r.ns * (32 * nw * 128) + 2 * (1024 * nw);
 }
 
 // Returns SC_EUNSUPPORTED when the shape does not suit this kernel (the caller falls
@@ -382,7 +553,7 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
         return SC_EUNSUPPORTED;
     // per-lane DMA offsets are 32-bit: x rows (M K 2 bytes) and a tile's weight rows
     if ((long long)M * K * 2 >= (1LL << 31) || (long long)K >= (1LL << 23)) return SC_EUNSUPPORTED;
-    const int mt = M <= 32 ? 1 : M <= 64 ? 2 : M <= 128 ? 4 : 8;
+    const int mt = M <= 16 ? 0 : M <= 32 ? 1 : M <= 64 ? 2 : M <= 128 ? 4 : 8;
     const int G = K / 64, nb = G / 8;
     const DeviceInfo &di = device_info();
     const int P = di.num_cus;
@@ -394,7 +565,7 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
     // ones).
     int nw = force_nw ? force_nw : 8;
     if (nw != 4 && nw != 8) return set_error(SC_EINVAL, "qgemm_band: waves %d (4 or 8)", nw);
-    if (!force_nw && (long)((N + 255) / 256) * nb < (mt == 1 ? 3L * P / 4 : 2L * P)) nw = 4;
+    if (!force_nw && (long)((N + 255) / 256) * nb < (mt <= 1 ? 3L * P / 4 : 2L * P)) nw = 4;
     if (mt > 2) nw = 4;
     const int tiles = (N + 32 * nw - 1) / (32 * nw);
     const int per_cu = band_lds(bits, mt, nw) <= 80 * 1024 ? 2 : 1;
@@ -424,12 +595,14 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
     }
     int rc;
     if (bits == 4) {
-        rc = mt == 1 ? launch_band_mt<4, 1>(a, nw, tiles, ksplit, stream)
+        rc = mt == 0 ? launch_band_mt<4, 0>(a, nw, tiles, ksplit, stream)
+           : mt == 1 ? launch_band_mt<4, 1>(a, nw, tiles, ksplit, stream)
            : mt == 2 ? launch_band_mt<4, 2>(a, nw, tiles, ksplit, stream)
            : mt == 4 ? launch_band_mt<4, 4>(a, nw, tiles, ksplit, stream)
                      : launch_band_mt<4, 8>(a, nw, tiles, ksplit, stream);
     } else {
-        rc = mt == 1 ? launch_band_mt<8, 1>(a, nw, tiles, ksplit, stream)
+        rc = mt == 0 ? launch_band_mt<8, 0>(a, nw, tiles, ksplit, stream)
+           : mt == 1 ? launch_band_mt<8, 1>(a, nw, tiles, ksplit, stream)
            : mt == 2 ? launch_band_mt<8, 2>(a, nw, tiles, ksplit, stream)
            : mt == 4 ? launch_band_mt<8, 4>(a, nw, tiles, ksplit, stream)
                      : launch_band_mt<8, 8>(a, nw, tiles, ksplit, stream);

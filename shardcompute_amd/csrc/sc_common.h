@@ -36,6 +36,12 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_vt));
 }
 
+// s + lo + hi of a bf16 pair, one v_dot2_f32_bf16
+__device__ __forceinline__ float add_pair_bf16(uint32_t pair, float s) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_vt, pair), __builtin_bit_cast(bf16x2_vt, 0x3F803F80u),
+                                           s, false);
+}
+
 // ---------------------------------------------------------------- exact elementwise math
 //
 // The kernels whose outputs are compared bit for bit (RMSNorm, residual add, SiLU

@@ -1,0 +1,40 @@
+"""The band kernel at up to 16 rows (16-row MFMA blocks, the x sums as fp32 MFMAs) and its
+stream's tail, against the float64 oracle.
+
+Codes stay exact on MFMA and scale and bias are applied per group in fp32, the decode GEMVs'
+rule, so the bound is theirs: 2 bf16 steps of the larger of the result and the product before
+the bias, plus 1e-5 of the largest result for the fp32 sums."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.bf16 import bf16_to_f32, f32_to_bf16
+from oracle.mlx_affine import quantize_bf16, quantized_matmul_f64
+from shardcompute_amd import _lib
+from tests.gpu_util import dev_bf16, dev_u32, host_u16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [1, 8, 15, 16])
+def test_band_up_to_16_rows(device, bits, M):
+    rng = np.random.default_rng(1600 + M + bits)
+    # one scale block (the tail alone), one weight row, ragged widths, several blocks
+    for K, N in [(512, 1), (512, 300), (1024, 257), (3584, 130), (8192, 96)]:
+        x = f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        wq, s, b = quantize_bf16((rng.standard_normal((N, K)) * 0.02).astype(np.float32), 64, bits)
+        bias = f32_to_bf16(rng.standard_normal(N).astype(np.float32) * 0.1) if N % 2 == 0 else None
+        prod = quantized_matmul_f64(x, wq, s, b, 64, bits)
+        ref = prod
+        if bias is not None:
+            ref = bf16_to_f32(f32_to_bf16(prod.astype(np.float32))).astype(np.float64) + bf16_to_f32(bias)[None, :]
+        for plan in [(0, 0), (8, 1), (4, 1), (8, 3), (4, 16)]:
+            print(f"band16 M={M} K={K} N={N} W{bits} plan={plan}", flush=True)
+            y = _lib.qmm(dev_bf16(x), dev_u32(wq), dev_bf16(s), dev_bf16(b),
+                         None if bias is None else dev_bf16(bias), bits=bits, band_plan=plan)
+            torch.cuda.synchronize()
+            got = bf16_to_f32(host_u16(y)).astype(np.float64)
+            _, e = np.frexp(np.maximum(np.abs(ref), np.abs(prod)))
+            bad = np.argwhere(np.abs(got - ref) > 2 * np.ldexp(1.0, e - 8) + 1e-5 * np.max(np.abs(ref)))
+            assert bad.size == 0, (plan, bad[0], got[tuple(bad[0])], ref[tuple(bad[0])])

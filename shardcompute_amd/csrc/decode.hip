@@ -221,18 +221,14 @@ rope_append_kernel(uint16_t *__restrict__ qkv, long qkv_stride, int S, int H, in
 // (one-token-per-wave scattering makes every 2-byte store touch its own line).
 // Same slots, same values, same bounds rule as rope_append_kernel.
 constexpr int VAPP_TOK = 64;
-__global__ void __launch_bounds__(256)
-v_append_kernel(const uint16_t *__restrict__ qkv, long qkv_stride, int S, int H, int Hkv, int D,
-                uint16_t *__restrict__ vt, int T_cap, const int32_t *__restrict__ cache_len, int pos_offset,
-                int table_len) {
-    __shared__ uint32_t tile[VAPP_TOK * (128 / 2 + 1)];   // token rows of D/2 + 1 words (odd: conflict-free columns)
-    const int s0 = blockIdx.x * VAPP_TOK, hk = blockIdx.y, b = blockIdx.z;
-    const int W = D / 2 + 1, cpt = D / 8;                  // words per LDS row, uint4 per token
-    const int base = cache_len[0];
+__device__ __forceinline__ void v_append_tile(uint32_t *tile, int s0, int hk, int b, const uint16_t *qkv,
+                                              long qkv_stride, int S, int H, int Hkv, int D, uint16_t *vt, int T_cap,
+                                              int base, int pos_offset, int table_len) {
+    const int W = D / 2 + 1, cpt = D / 8;                  // words per LDS row (odd: conflict-free columns), uint4 per token
     for (int i = threadIdx.x; i < VAPP_TOK * cpt; i += 256) {
         const int t = i / cpt, c = i - t * cpt;
         if (s0 + t < S) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(qkv + (size_t)(b * S + s0 + t) * qkv_stride +
+            const uint4 v = *reinterpret_cast<const uint4 *>(qkv + ((size_t)b * S + s0 + t) * qkv_stride +
                                                              (size_t)(H + Hkv + hk) * D + 8 * c);
             uint32_t *row = tile + t * W + 4 * c;
             row[0] = v.x; row[1] = v.y; row[2] = v.z; row[3] = v.w;
@@ -247,6 +243,76 @@ v_append_kernel(const uint16_t *__restrict__ qkv, long qkv_stride, int S, int H,
     for (int d = w * dpw; d < (w + 1) * dpw; ++d) {
         const uint32_t word = tile[lane * W + (d >> 1)];
         vc[(size_t)d * T_cap] = (uint16_t)((d & 1) ? (word >> 16) : (word & 0xFFFFu));
+    }
+}
+
+__global__ void __launch_bounds__(256)
+v_append_kernel(const uint16_t *__restrict__ qkv, long qkv_stride, int S, int H, int Hkv, int D,
+                uint16_t *__restrict__ vt, int T_cap, const int32_t *__restrict__ cache_len, int pos_offset,
+                int table_len) {
+    __shared__ uint32_t tile[VAPP_TOK * (128 / 2 + 1)];
+    v_append_tile(tile, (int)blockIdx.x * VAPP_TOK, blockIdx.y, blockIdx.z, qkv, qkv_stride, S, H, Hkv, D, vt, T_cap,
+                  cache_len[0], pos_offset, table_len);
+}
+
+// rope_append for many new positions, one launch: the first v_tiles workgroups append v
+// (v_append_tile), the others rotate four tokens each, a wave per token.  A lane takes 8
+// dims of a head's first half and the matching 8 of its second (16-byte loads and stores;
+// D / 16 lanes a head, so a wave's heads are contiguous) and keeps the token's cos and sin
+// of its dims for all its heads.  Bound by memory latency and launches at these sizes:
+// 2048 tokens of 32 + 8 heads of 128 17.9 + 5.6 us (one 2-byte element per lane, v in a
+// second launch) -> 9.6, 3 x 701 of 32 + 4 heads of 64 15.7 + 4.4 -> 7.7, 16 x 2048 344 -> 166
+// (4.9 TB/s).  The arithmetic is rope_append_kernel's, element by element.
+template <int D>
+__global__ void __launch_bounds__(256)
+rope_append_wide_kernel(uint16_t *__restrict__ qkv, long qkv_stride, int tokens, int S, int H, int Hkv,
+                        const float *__restrict__ cos_t, const float *__restrict__ sin_t, uint16_t *__restrict__ kc,
+                        uint16_t *__restrict__ vt, int T_cap, const int32_t *__restrict__ cache_len, int pos_offset,
+                        int table_len, int v_tiles, int tiles_s) {
+    __shared__ uint32_t tile[VAPP_TOK * (D / 2 + 1)];
+    const int base = cache_len[0];
+    if ((int)blockIdx.x < v_tiles) {
+        const int t = (int)blockIdx.x / tiles_s;           // b Hkv + hk
+        v_append_tile(tile, ((int)blockIdx.x - t * tiles_s) * VAPP_TOK, t % Hkv, t / Hkv, qkv, qkv_stride, S, H, Hkv, D,
+                      vt, T_cap, base, pos_offset, table_len);
+        return;
+    }
+    constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;   // lanes a head, heads a wave at a time
+    const int tok = ((int)blockIdx.x - v_tiles) * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (tok >= tokens) return;
+    const int b = tok / S, s = tok - b * S;
+    const int pos = base + s, rpos = pos + pos_offset;
+    if (pos < 0 || pos >= T_cap || rpos < 0 || rpos >= table_len) return;   // as rope_append_kernel
+    const int i0 = 8 * (lane % LPH);
+    float c[8], sn[8];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const float4 cv = *reinterpret_cast<const float4 *>(cos_t + (size_t)rpos * HALF + i0 + 4 * q);
+        const float4 sv = *reinterpret_cast<const float4 *>(sin_t + (size_t)rpos * HALF + i0 + 4 * q);
+        c[4 * q] = cv.x; c[4 * q + 1] = cv.y; c[4 * q + 2] = cv.z; c[4 * q + 3] = cv.w;
+        sn[4 * q] = sv.x; sn[4 * q + 1] = sv.y; sn[4 * q + 2] = sv.z; sn[4 * q + 3] = sv.w;
+    }
+    uint16_t *row = qkv + (size_t)tok * qkv_stride + i0;
+#pragma unroll 4
+    for (int head = lane / LPH; head < H + Hkv; head += HPW) {
+        uint16_t *hp = row + (size_t)head * D;
+        const uint4 a1 = *reinterpret_cast<const uint4 *>(hp), a2 = *reinterpret_cast<const uint4 *>(hp + HALF);
+        uint32_t o1[4], o2[4];
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            float r1[2], r2[2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const float x1 = bfe(a1, e + f), x2 = bfe(a2, e + f);
+                r1[f] = add_rn(mul_rn(x1, c[e + f]), mul_rn(-x2, sn[e + f]));
+                r2[f] = add_rn(mul_rn(x2, c[e + f]), mul_rn(x1, sn[e + f]));
+            }
+            o1[e / 2] = pack_bf16x2(r1[0], r1[1]);
+            o2[e / 2] = pack_bf16x2(r2[0], r2[1]);
+        }
+        uint16_t *dst = head < H ? hp : kc + (((size_t)b * Hkv + (head - H)) * T_cap + pos) * D + i0;
+        *reinterpret_cast<uint4 *>(dst) = make_uint4(o1[0], o1[1], o1[2], o1[3]);
+        *reinterpret_cast<uint4 *>(dst + HALF) = make_uint4(o2[0], o2[1], o2[2], o2[3]);
     }
 }
 
@@ -1046,8 +1112,22 @@ int launch_rope_append(uint16_t *qkv, long qkv_stride, long B, long S, long H, l
     if (T_cap <= 0 || table_len <= 0 || pos_offset < 0 || T_cap > 0x7FFFFFFFL || table_len > 0x7FFFFFFFL ||
         pos_offset > 0x7FFFFFFFL)
         return set_error(SC_EINVAL, "rope_append: bad capacity/table/offset");
-    // many positions: v through v_append_kernel (64 tokens a workgroup), when its
-    // 16-byte row loads are aligned
+    // many positions (16 to fill a v tile's lines), head_dim 128 or 64 and 16-byte aligned
+    // rows, tables and cache: the one-launch kernel; otherwise a wave per head and token
+    const long tiles_s = (S + VAPP_TOK - 1) / VAPP_TOK;
+    if (S >= 16 && (D == 128 || D == 64) && qkv_stride % 8 == 0 &&
+        ((uintptr_t)qkv | (uintptr_t)kc | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16 == 0 &&
+        B * Hkv * tiles_s + (B * S + 3) / 4 <= 0x7FFFFFFFL) {
+        const int v_tiles = (int)(B * Hkv * tiles_s);
+        const dim3 grid((unsigned)(v_tiles + (B * S + 3) / 4));
+        auto kern = D == 128 ? rope_append_wide_kernel<128> : rope_append_wide_kernel<64>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, qkv, qkv_stride, (int)(B * S), (int)S, (int)H, (int)Hkv,
+                           cos_t, sin_t, kc, vt, (int)T_cap, cache_len, (int)pos_offset, (int)table_len, v_tiles,
+                           (int)tiles_s);
+        SC_HIP_CHECK(hipGetLastError());
+        return SC_OK;
+    }
+    // (other head dims: v through v_append_kernel, when its 16-byte row loads are aligned)
     const bool tiled_v = S >= 16 && D % 8 == 0 && D <= 128 && qkv_stride % 8 == 0 && (uintptr_t)qkv % 16 == 0;
     const int v_heads = tiled_v ? 0 : (int)Hkv;
     hipLaunchKernelGGL(rope_append_kernel, dim3((unsigned)(B * S), (unsigned)((H + Hkv + v_heads + 3) / 4)), dim3(256),
@@ -1056,9 +1136,9 @@ int launch_rope_append(uint16_t *qkv, long qkv_stride, long B, long S, long H, l
                        (int)table_len, v_heads);
     SC_HIP_CHECK(hipGetLastError());
     if (tiled_v) {
-        hipLaunchKernelGGL(v_append_kernel, dim3((unsigned)((S + VAPP_TOK - 1) / VAPP_TOK), (unsigned)Hkv, (unsigned)B),
-                           dim3(256), 0, stream, qkv, qkv_stride, (int)S, (int)H, (int)Hkv, (int)D, vt, (int)T_cap,
-                           cache_len, (int)pos_offset, (int)table_len);
+        hipLaunchKernelGGL(v_append_kernel, dim3((unsigned)tiles_s, (unsigned)Hkv, (unsigned)B), dim3(256), 0, stream,
+                           qkv, qkv_stride, (int)S, (int)H, (int)Hkv, (int)D, vt, (int)T_cap, cache_len,
+                           (int)pos_offset, (int)table_len);
         SC_HIP_CHECK(hipGetLastError());
     }
     return SC_OK;

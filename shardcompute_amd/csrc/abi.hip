@@ -28,6 +28,9 @@ int64_t qgemm_dense_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                        const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                        int swiglu_half, void *ws, int64_t ws_bytes);
+int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
+                     const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
+                     int swiglu_half, bool no_alloc);
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                       bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr);
@@ -203,6 +206,10 @@ static int qmm_dispatch(const uint16_t *x, const uint32_t *wq, const uint16_t *s
         rc = launch_qgemm_dense(x, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, 0, wsp.ws, wsp.bytes);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
+    if (path == SC_QMM_PATH_AUTO && M > 160) {
+        rc = launch_qgemm_mid(x, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, 0, no_alloc);
+        if (rc != SC_EUNSUPPORTED) return rc;
+    }
     if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K, bits) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
                                                                                     : SC_QMM_PATH_GEMM;
     if (path == SC_QMM_PATH_BAND) {
@@ -314,6 +321,10 @@ static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw,
     if (M > 8 && M <= 32) {
         // the 9-32-row GEMV's split-K pass applies silu(gate) * up itself
         rc = launch_qgemv16(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half);
+        if (rc != SC_EUNSUPPORTED) return rc;
+    }
+    if (M > 160) {
+        rc = launch_qgemm_mid(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, (int)swiglu_half, false);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
     if (M > 32) {

@@ -39,6 +39,7 @@
 //   weight tiles in its L2.
 #include "sc_common.h"
 #include "dma_util.h"
+#include "gemm_store.h"
 
 #include <type_traits>
 #include <utility>
@@ -284,37 +285,7 @@ qgemm_dense_kernel(DenseArgs a) {
                                  cvt_pk_bf16(acc[i][2 * p][2], acc[i][2 * p][3]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][0], acc[i][2 * p + 1][1]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][2], acc[i][2 * p + 1][3])};
-                if (!FAST && a.bias) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        // SwiGLU: columns 2j, 2j + 1 are gate j and up j
-                        const int c0 = SWIGLU ? (c >> 1) + e : c + 2 * e, c1 = SWIGLU ? a.swiglu_i + c0 : c0 + 1;
-                        if (n + 2 * e < N)
-                            o[e] = cvt_pk_bf16(bf2f(o[e] & 0xFFFFu) + bf2f(a.bias[c0]),
-                                               bf2f(o[e] >> 16) + (n + 2 * e + 1 < N ? bf2f(a.bias[c1]) : 0.f));
-                    }
-                }
-                if (SWIGLU) {
-                    float s[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) s[e] = silu_mul_f(bf2f(o[e] & 0xFFFFu), bf2f(o[e] >> 16));
-                    uint16_t *d = yr + (c >> 1);
-                    if (FAST) {
-                        *reinterpret_cast<uint2 *>(d) = make_uint2(cvt_pk_bf16(s[0], s[1]), cvt_pk_bf16(s[2], s[3]));
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (n + 2 * e < N) d[e] = (uint16_t)f2bf(s[e]);
-                    }
-                } else if (FAST) {
-                    *reinterpret_cast<uint4 *>(yr + c) = make_uint4(o[0], o[1], o[2], o[3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (n + 2 * e < N) yr[c + 2 * e] = (uint16_t)o[e];
-                        if (n + 2 * e + 1 < N) yr[c + 2 * e + 1] = (uint16_t)(o[e] >> 16);
-                    }
-                }
+                store_cols8<FAST, SWIGLU>(o, yr, c, n, N, a.bias, a.swiglu_i);
             }
         }
     };

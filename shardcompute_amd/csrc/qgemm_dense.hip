@@ -34,9 +34,9 @@
 //   MFMA): two of them in a slot outlast the 16 cycles of the MFMA (2-3 %).
 // * A 4- or 5-stage ring of 32-k stages (more bytes in flight, a barrier per 32) was
 //   5 % slower, 32x32x16 MFMAs 3-5 %, DMA spread over both k-steps 8 %.
-// * Tiles are dealt to the XCDs in contiguous runs, in column order inside groups of
-//   GROUP_M row tiles, so that the 32 tiles an XCD works on share 4 x tiles and 8
-//   weight tiles in its L2.
+// * Tiles are dealt to the XCDs in contiguous runs, in column order inside groups of 4 or 8
+//   row tiles, so that the 32 tiles an XCD works on share 4 x tiles and 8 weight tiles
+//   (or 8 and 4) in its L2.
 #include "sc_common.h"
 #include "dma_util.h"
 #include "gemm_store.h"
@@ -53,7 +53,6 @@ namespace {
 constexpr int BK = 64;                    // k per stage: one 128-byte row of LDS
 constexpr int ROW_BYTES = BK * 2;
 constexpr int XCDS = 8;
-constexpr int GROUP_M = 4;
 constexpr int BM = 256;
 // columns of weights dequantized at a time: the workspace holds at most this many bytes
 constexpr int64_t WS_MAX_BYTES = 256ll << 20;
@@ -69,6 +68,7 @@ struct DenseArgs {
     int swiglu_i;             // I > 0: columns 2j, 2j + 1 are gate j and up j; y receives act [M, I]
     int vec;                  // rows of y are aligned for 16-byte (SwiGLU: 8-byte) stores
     int mt, nt, tiles;
+    int group_m;              // row tiles a run of tiles walks before the next column
 };
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -148,8 +148,8 @@ qgemm_dense_kernel(DenseArgs a) {
     const int per = (int)(gridDim.x / XCDS);
     const int tile = (int)(blockIdx.x % XCDS) * per + (int)(blockIdx.x / XCDS);
     if (tile >= a.tiles) return;
-    const int grp = tile / (GROUP_M * a.nt), first = grp * GROUP_M;
-    const int rows = min(GROUP_M, a.mt - first), in = tile - grp * GROUP_M * a.nt;
+    const int grp = tile / (a.group_m * a.nt), first = grp * a.group_m;
+    const int rows = min(a.group_m, a.mt - first), in = tile - grp * a.group_m * a.nt;
     const int m0 = (first + in % rows) * BM, n0 = in / rows * BN;
 
     // DMA instruction i of this wave covers 8 tile rows; lane l lands at row l / 8,
@@ -348,6 +348,10 @@ static int launch_dense_cols(const DenseArgs &full, int n0, int nc, hipStream_t 
     const int64_t tiles = (int64_t)a.mt * a.nt;
     if (tiles > 0x7FFFFFF0) return set_error(SC_EINVAL, "qgemm_dense: grid too large");
     a.tiles = (int)tiles;
+    // 8 row tiles where the launch is one round, 4 otherwise (measured, 4 -> 8: 2048 x 4096 x
+    // 4096 73.4 -> 70.3 us, x 6144 94.2 -> 91.4, but 2048 x 28672 x 4096 440 -> 444; 2 is
+    // slower everywhere, 8192 x 7168 x 8192 689 -> 739)
+    a.group_m = tiles <= device_info().num_cus ? 8 : 4;
     constexpr int LDS = 2 * (BM + BN) * ROW_BYTES;
     auto kern = qgemm_dense_kernel<BN, WGM, WGN>;
     static bool configured = false;

@@ -31,6 +31,7 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
 int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                      const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                      int swiglu_half, bool no_alloc);
+int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits);
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                       bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr);
@@ -173,10 +174,13 @@ static int check_qmm(const void *x, const void *wq, const void *s, const void *b
 // kernels compute 32 rows and the band's stream is the faster (8B gate|up at 20, 24
 // and 32 rows 28, 31, 30 against 32, 34, 34 us on the GEMV; the 8B lm_head at 32 rows
 // 99 against 119 us); 9-16 rows where the 16-column GEMV's K splits or x staging cost
-// more than the band's stream: K above 4096, or up to 16384 weight rows at 4 bits and
-// 65536 at 8 (TinyLlama gate|up at 16 rows 11.5 against 12.0 us, W8 12.2 against 15.0; 8B
-// gate|up W8 34.0 against 38.5, W4 24.6 against 24.4; the 8B lm_head 77 against 70, W8 139
-// against 135);
+// more than the band's stream: K above 4096, up to 8192 weight rows, or up to 16384 at
+// 4 bits and 65536 at 8 (TinyLlama gate|up at 16 rows 11.5 against 12.0 us, W8 12.2 against
+// 15.0; 8B gate|up W8 34.0 against 38.5, W4 24.6 against 24.4; the 8B lm_head 77 against 70,
+// W8 139 against 135).  Above 8192 rows of K up to 4096 only where the scratch is needed no
+// more than on the GEMV: the band's partials fit the allocation-free array, so that
+// sc_qmm_bf16_noalloc stays bit-equal, and the GEMV would split K as well (it does below
+// 8 tiles of 16 rows a CU; from there on it needs no scratch);
 // and 8 rows with K of 4096 or more (8B q|k|v, gate|up, down 10, 24, 16 against 13,
 // 25, 26 us on the 8-row GEMV; K = 2048 is a tie).  4-7 rows, and 8 rows of a smaller K, are
 // up to 1.6 times faster here too (8B down at 4 rows 16 against 25 us), but stay on the GEMV:
@@ -185,7 +189,11 @@ static int check_qmm(const void *x, const void *wq, const void *s, const void *b
 static bool band_first(int64_t M, int64_t N, int64_t K, int bits) {
     if (M > 32) return M <= 160;
     if (M == 8) return K >= 4096;
-    return M > 16 || (M > 8 && (K > 4096 || N <= (bits == 4 ? 16384 : 65536)));
+    if (M > 16 || (M > 8 && (K > 4096 || N <= 8192))) return true;
+    if (M <= 8 || N > (bits == 4 ? 16384 : 65536) || K % 512) return false;
+    const int64_t partials = qgemm_band_partials(M, N, K, bits);
+    return partials * (int64_t)sizeof(float) <= (int64_t)SC_QMM_NOALLOC_SCRATCH_BYTES &&
+           (!partials || (N + 15) / 16 < 8 * (int64_t)device_info().num_cus);
 }
 
 // The caller's workspace of a call (none: ws null), for the products whose weights are

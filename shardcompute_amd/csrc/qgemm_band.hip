@@ -534,6 +534,39 @@ static int band_lds(int bits, int mt, int nw) {
     return r.nx * band_xb(mt) + r.ns * (32 * nw * 128) + 2 * (1024 * nw);
 }
 
+static int band_mt(int M) { return M <= 16 ? 0 : M <= 32 ? 1 : M <= 64 ? 2 : M <= 128 ? 4 : 8; }
+
+struct BandPlan {
+    int nw, tiles, ksplit, bps;                          // bps: scale/bias blocks per split
+};
+
+// 8-wave workgroups (256 rows) unless too few tiles would be left to fill the CUs even
+// with every scale/bias block a split of its own (twice over above 32 rows, three quarters
+// over up to 32: measured on the decode shapes); then the K splits that bring the
+// workgroups to about one round (two per CU for the small 4-wave ones).
+static BandPlan plan_band(int M, int N, int K, int bits, int force_nw, int force_split) {
+    const int mt = band_mt(M), nb = K / 512;
+    const int P = device_info().num_cus;
+    BandPlan p;
+    p.nw = force_nw ? force_nw : 8;
+    if (!force_nw && (long)((N + 255) / 256) * nb < (mt <= 1 ? 3L * P / 4 : 2L * P)) p.nw = 4;
+    if (mt > 2) p.nw = 4;
+    p.tiles = (N + 32 * p.nw - 1) / (32 * p.nw);
+    const int per_cu = band_lds(bits, mt, p.nw) <= 80 * 1024 ? 2 : 1;
+    int ks = force_split ? force_split : (int)((P * per_cu + p.tiles / 2) / p.tiles);
+    if (ks < 1) ks = 1;
+    if (ks > nb) ks = nb;
+    p.bps = (nb + ks - 1) / ks;
+    p.ksplit = (nb + p.bps - 1) / p.bps;
+    return p;
+}
+
+// Floats of split-K partials that a product on this kernel takes from the scratch (0: none).
+int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits) {
+    const BandPlan p = plan_band((int)M, (int)N, (int)K, bits, 0, 0);
+    return p.ksplit > 1 ? p.ksplit * M * N : 0;
+}
+
 // Returns SC_EUNSUPPORTED when the shape does not suit this kernel (the caller falls
 // back).  force_nw / force_split (0 = automatic) pin the plan for measurements.
 // no_alloc: the split-K partials go to the allocation-free scratch array (shapes that
@@ -553,27 +586,12 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
         return SC_EUNSUPPORTED;
     // per-lane DMA offsets are 32-bit: x rows (M K 2 bytes) and a tile's weight rows
     if ((long long)M * K * 2 >= (1LL << 31) || (long long)K >= (1LL << 23)) return SC_EUNSUPPORTED;
-    const int mt = M <= 16 ? 0 : M <= 32 ? 1 : M <= 64 ? 2 : M <= 128 ? 4 : 8;
-    const int G = K / 64, nb = G / 8;
-    const DeviceInfo &di = device_info();
-    const int P = di.num_cus;
-
-    // Plan: 8-wave workgroups (256 rows) unless too few tiles would be left to fill the
-    // CUs even with every scale/bias block a split of its own (twice over above 32 rows,
-    // three quarters over up to 32: measured on the decode shapes); then the K splits
-    // that bring the workgroups to about one round (two per CU for the small 4-wave
-    // ones).
+    const int mt = band_mt(M), G = K / 64;
     int nw = force_nw ? force_nw : 8;
     if (nw != 4 && nw != 8) return set_error(SC_EINVAL, "qgemm_band: waves %d (4 or 8)", nw);
-    if (!force_nw && (long)((N + 255) / 256) * nb < (mt <= 1 ? 3L * P / 4 : 2L * P)) nw = 4;
-    if (mt > 2) nw = 4;
-    const int tiles = (N + 32 * nw - 1) / (32 * nw);
-    const int per_cu = band_lds(bits, mt, nw) <= 80 * 1024 ? 2 : 1;
-    int ksplit = force_split ? force_split : (int)((P * per_cu + tiles / 2) / tiles);
-    if (ksplit < 1) ksplit = 1;
-    if (ksplit > nb) ksplit = nb;
-    const int bps = (nb + ksplit - 1) / ksplit;          // blocks per split
-    ksplit = (nb + bps - 1) / bps;
+    const BandPlan p = plan_band(M, N, K, bits, force_nw, force_split);
+    nw = p.nw;
+    const int tiles = p.tiles, ksplit = p.ksplit, bps = p.bps;
 
     BandArgs a;
     a.x = x; a.wq = reinterpret_cast<const uint8_t *>(wq); a.s = s; a.b = b; a.bias = bias; a.y = y;

@@ -11,7 +11,7 @@ import torch
 from oracle.bf16 import bf16_to_f32, f32_to_bf16
 from oracle.mlx_affine import quantize_bf16, quantized_matmul_f64
 from shardcompute_amd import _lib
-from tests.gpu_util import dev_bf16, dev_u32, host_u16
+from tests.gpu_util import dev_bf16, dev_u32, host_u16, host_u32
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,28 @@ def test_band_up_to_16_rows(device, bits, M):
             _, e = np.frexp(np.maximum(np.abs(ref), np.abs(prod)))
             bad = np.argwhere(np.abs(got - ref) > 2 * np.ldexp(1.0, e - 8) + 1e-5 * np.max(np.abs(ref)))
             assert bad.size == 0, (plan, bad[0], got[tuple(bad[0])], ref[tuple(bad[0])])
+
+
+@pytest.mark.parametrize("bits,M,N,K", [
+    (4, 16, 8192, 1024), (4, 16, 11264, 2048), (4, 16, 14000, 4096), (4, 9, 16384, 512),  # fit / fit / exceed / unsplit
+    (8, 16, 32752, 1024), (8, 9, 32768, 1024), (8, 16, 22000, 4096), (8, 9, 43528, 1024)])
+def test_wide_products_of_9_to_16_rows_need_no_more_scratch(device, bits, M, N, K):
+    """The allocation-free entry gives sc_qmm_bf16's bits on either side of every line of
+    the 9-16-row rule (8192, 16384 and 65536 weight rows, the partials' limit, the sizes
+    that the GEMV does not split)."""
+    rng = np.random.default_rng(N + K)
+    x = dev_bf16(f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32)))
+    per = 8 if bits == 4 else 4
+    wq = dev_u32(rng.integers(0, 2**32, (N, K // per), dtype=np.uint32))
+    s = dev_bf16(f32_to_bf16(rng.uniform(0.001, 0.01, (N, K // 64)).astype(np.float32)))
+    b = dev_bf16(f32_to_bf16(rng.uniform(-0.05, 0.05, (N, K // 64)).astype(np.float32)))
+    y = _lib.qmm(x, wq, s, b, None, bits=bits)
+    y2 = _lib.qmm(x, wq, s, b, None, bits=bits, no_alloc=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    cols = np.r_[0:16, N // 2:N // 2 + 16, N - 16:N]
+    ref = quantized_matmul_f64(host_u16(x), host_u32(wq)[cols], host_u16(s)[cols],
+                               host_u16(b)[cols], 64, bits)
+    got = bf16_to_f32(host_u16(y)).astype(np.float64)[:, cols]
+    _, e = np.frexp(np.abs(ref))
+    assert np.all(np.abs(got - ref) <= 2 * np.ldexp(1.0, e - 8) + 1e-5 * np.max(np.abs(ref)))

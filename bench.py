@@ -535,19 +535,20 @@ def bench_lm_head_m64(reps=10):
             "frac_hbm": round(gbs / HBM_PEAK_GBS, 4), "TFLOPs": round(tf, 1)}
 
 
-def qmm_kernel_label(M, N, K, bits, cus=256):
+def qmm_kernel_label(M, N, K, cus=256):
     """The kernel the automatic path takes for an M x K -> N product (the choice
-    csrc/abi.hip, csrc/qgemm_dense.hip and csrc/qgemm.hip make, restated for the sweep's
-    labels)."""
+    csrc/abi.hip, csrc/qgemm_dense.hip, csrc/qgemm_mid.hip and csrc/qgemm.hip make, restated
+    for the sweep's labels: none of its sizes has 9-16 rows)."""
     from shardcompute_amd import _lib
     if _lib.load().sc_qmm_workspace_bytes(M, N, K) > 0:
         return "dequantize + dense gemm"
-    band = K % 512 == 0 and (M <= 160 if M > 32 else K >= 4096 if M == 8 else
-                             M > 16 or M > 8 and (K > 4096 or N <= (16384 if bits == 4 else 65536)))
-    if band:
+    if K % 512 == 0 and (M <= 160 if M > 16 else M == 8 and K >= 4096):
         return "band"
     if M <= 32:
         return "gemv"
+    tiles128 = ((M + 127) // 128) * ((N + 127) // 128)
+    if M > 160 and K % 512 == 0 and tiles128 <= (cus if K < 4096 else cus // 4):
+        return "gemm, 128 x 128 tiles"
     tiles256 = ((M + 255) // 256) * ((N + 255) // 256)
     return "gemm, K split" if 4 * tiles256 <= cus and K // 64 >= 64 else "gemm"
 
@@ -609,7 +610,7 @@ def bench_qmm_sweep(reps=5):
                 us = e0.elapsed_time(e1) * 1e3 / (reps * copies)
                 nbytes = qmm_bytes(M, N, K, bits)
                 flops = 2.0 * M * N * K
-                kernel = qmm_kernel_label(M, N, K, bits)
+                kernel = qmm_kernel_label(M, N, K)
                 row = {"bits": bits, "M": M, "K": K, "N": N, "kernel": kernel, "gpu_us": round(us, 2)}
                 if M <= 32:
                     gbs = nbytes / (us * 1e-6) / 1e9

@@ -15,7 +15,8 @@
  *    holds a message (thread-local, valid until the next failing call).
  *  - The kernels allocate nothing per call.  The split-K path of sc_qmm_bf16 (and of
  *    the products inside sc_qmm_rmsnorm_bf16 / sc_qmm_swiglu_bf16 / sc_qmm_add_rmsnorm_bf16:
- *    9-160 rows, and larger products whose 256-wide tiles fill at most half the GPU) uses a
+ *    8-160 rows, and larger products whose 256-wide tiles fill at most a quarter of the GPU
+ *    over K >= 4096) uses a
  *    library-owned scratch per device, allocated on first need and grown (with a
  *    device synchronisation) when a larger shape arrives: calls that overlap on one
  *    device (concurrent streams) race on it, and the first call of a new largest
@@ -35,7 +36,9 @@ extern "C" {
 
 /* Kernel selection for sc_qmm_bf16_path. */
 #define SC_QMM_PATH_AUTO 0 /* M <= 16: GEMV or band kernel (8-16 rows, by shape);
-                              17-160: band kernel; above: GEMM                  */
+                              17-160: band kernel; above: 128x128-tile GEMM (few
+                              tiles) or GEMM; with a workspace (the _ws entries):
+                              dequantize once, then the dense GEMM              */
 #define SC_QMM_PATH_GEMV 1 /* fused dequant-GEMV (decode batches, M <= 32)      */
 #define SC_QMM_PATH_GEMM 2 /* LDS-staged dequant -> bf16 MFMA GEMM (prefill)     */
 #define SC_QMM_PATH_BAND 3 /* weight-streaming band kernel (M <= 256)            */
@@ -121,8 +124,8 @@ int sc_qmm_bf16_band(const uint16_t *x, const uint32_t *wq, const uint16_t *scal
  * hipMalloc: code under HIP graph capture, tight serving loops, harnesses that
  * forbid allocation.  No counterpart in the reference (mx.quantized_matmul
  * allocates its output; this entry point allocates nothing at all).  Same
- * arguments, kernels and results as sc_qmm_bf16, bit for bit.  Where the 9-160-row
- * band kernel or the 9-32-row GEMV splits K across workgroups, its fp32 partials go
+ * arguments, kernels and results as sc_qmm_bf16, bit for bit.  Where the 8-160-row
+ * band kernel, the 9-32-row GEMV or a GEMM splits K across workgroups, its fp32 partials go
  * to a file-scope device array of SC_QMM_NOALLOC_SCRATCH_BYTES (one per GPU, held
  * until the process ends) instead of the library's growable buffer.  A shape whose
  * partials (splits * M * N floats) exceed it runs on the next kernel that needs no

@@ -35,11 +35,13 @@ __device__ __forceinline__ uint4 perm_w4x(uint4 v) {
 // 16 bytes per active lane from global `g` to LDS byte address lds_base + 16 * lane.
 // The instruction takes its LDS base from M0, which this block sets itself; the
 // kernel has no other M0 user (no LDS-DMA builtins, no indirect register access),
-// so declaring the clobber is all the compiler needs (it warns regardless).
+// so declaring the clobber is all the compiler needs (it warns regardless).  The DMA
+// needs one wait state after the scalar write of M0; the compiler puts an s_nop there
+// itself for its builtin, but sees nothing inside an asm block.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds_base))
                  : "memory", "m0");
@@ -47,7 +49,7 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
 // The same with a wave-uniform 64-bit base in SGPRs and a 32-bit byte offset per
 // lane (the SADDR form: no 64-bit address per lane in VGPRs).
 __device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(voff), "s"(sbase), "s"(__builtin_amdgcn_readfirstlane(lds_base))
                  : "memory", "m0");

@@ -416,8 +416,8 @@ static int launch_fa(const FaArgs &f, long wgs, hipStream_t stream) {
 
 // Launches attn_prefill_kernel when the shape suits it (head_dim 128 or 64, the GQA ratio
 // dividing 128, 16-byte aligned Vt, at least 128 / R new positions: one workgroup's
-// columns) and returns SC_OK; returns 1, launching nothing, when it does not.  The
-// choice does not depend on the batch size, so that a sequence's result is the same
+// columns, a positive scale) and returns SC_OK; returns 1, launching nothing, when it
+// does not.  The choice does not depend on the batch size, so that a sequence's result is the same
 // alone and in a batch (every column's arithmetic is its own).  The caller has
 // checked the shape, strides and pointers as launch_attention does.  mask / ms: the
 // additive mask and its strides (b, h, s, t), or null.
@@ -426,6 +426,10 @@ int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, co
                         long D, float scale, hipStream_t stream, const float *mask, const long *ms) {
     const long R = H / Hkv;
     if ((D != 128 && D != 64) || FA_COLS % R != 0 || ((uintptr_t)vt % 16) != 0) return 1;
+    // The maximum is taken of the unscaled scores, and a mask is divided by the scale: right
+    // for a positive scale whose reciprocal is a normal number.  Any other scale (zero,
+    // negative, NaN, the ends of the range) is attn_kernel's, which scales the scores first.
+    if (!(scale >= 1e-30f && scale <= 1e30f)) return 1;
     // head_dim 64: few query rows over many keys stay on attn_kernel, which splits the keys
     // over workgroups (a workgroup here takes ~1 us per 64 keys).  Measured, one sequence,
     // 32 q heads on 4 kv heads, attn_kernel -> here: 128 positions after 1500 16 -> 26 us,

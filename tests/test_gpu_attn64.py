@@ -63,3 +63,31 @@ def test_prefill_attention_head_dim_64(device, B, S, H, Hkv, past, T_cap, masked
     got = out.view(B, S, H, D).transpose(1, 2).double()
     assert torch.isfinite(got).all()
     assert (got - ref).abs().max() <= 1e-2 * ref.abs().max()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("masked", [False, True])
+def test_prefill_softmax_sum_is_fp32(device, D, masked):
+    """The probabilities meet V in bf16, their sum is that of the fp32 values.  One key block
+    (no running maximum), so the result is known to its last bit but for the few elements
+    whose probabilities lie within the scores' fp32 error (~2^-20) of a bf16 rounding
+    boundary, ~1e-3 of them; a sum of the rounded values moves 4-5 % of them."""
+    S, H, past = 40, 8, 24
+    T = past + S
+    g = torch.Generator(device="cuda")
+    g.manual_seed(D)
+    q = torch.randn((S, H * D), generator=g, device="cuda").to(torch.bfloat16)
+    kc = torch.randn((1, 1, T, D), generator=g, device="cuda").to(torch.bfloat16)
+    vt = torch.randn((1, 1, D, T), generator=g, device="cuda").to(torch.bfloat16)
+    mask = torch.randn((1, 1, 1, T), generator=g, device="cuda") if masked else None
+    cnt = torch.tensor([past, 0], dtype=torch.int32, device="cuda")
+    out = _lib.attention(q, 1, S, H, 1, D, kc, vt, cnt, 1 / math.sqrt(D), mask=mask, n_keys=T).view(S, H, D)
+    hidden = torch.arange(T, device="cuda")[None] > torch.arange(past, T, device="cuda")[:, None]
+    s = q.view(S, H, D).transpose(0, 1).double() @ kc[0, 0].double().T.contiguous() / math.sqrt(D)
+    if masked:
+        s = s + mask[0].double()
+    s = s.masked_fill(hidden, -math.inf)
+    p = torch.exp(s - s.amax(-1, keepdim=True))
+    o = p.float().to(torch.bfloat16).double() @ vt[0, 0].double().T.contiguous()
+    exact = (o / p.sum(-1, keepdim=True)).float().to(torch.bfloat16)
+    assert (out.transpose(0, 1) != exact).double().mean() <= 0.01

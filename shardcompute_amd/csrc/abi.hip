@@ -18,7 +18,7 @@ int launch_qgemv_dma(const uint16_t *x, const uint32_t *wq, const uint16_t *s, c
 bool qgemv_dma_eligible(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b, int M, int K);
 int launch_qgemv16(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b, const uint16_t *bias,
                    uint16_t *y, int M, int N, int K, int bits, hipStream_t stream, bool no_alloc, int swiglu_half = 0,
-                   SplitKeep *keep = nullptr);
+                   SplitKeep *keep = nullptr, uint16_t *gate_up = nullptr);
 int launch_qgemv_skinny(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                         const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream);
 int launch_qgemm_mfma(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
@@ -34,7 +34,8 @@ int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, c
 int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits);
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
-                      bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr);
+                      bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr,
+                      uint16_t *gate_up = nullptr);
 int launch_vocab_gather(const void *ids, int ids_is_int64, int64_t T, const uint16_t *table, int64_t v_local,
                         int64_t D, int64_t vocab_start, uint16_t *out, hipStream_t stream);
 int launch_qembed_gather(const void *ids, int ids_is_int64, int64_t T, const uint32_t *wq, const uint16_t *s,
@@ -64,7 +65,6 @@ int launch_attention(const uint16_t *q, long q_stride, const uint16_t *kc, const
                      const int32_t *cache_len, uint16_t *out, long out_stride, long B, long S, long H, long Hkv,
                      long D, float scale, void *workspace, long workspace_bytes, hipStream_t stream,
                      const float *mask, const long *mask_strides);
-int launch_silu_mul(const uint16_t *gu, long rows, long I, uint16_t *out, hipStream_t stream);
 int launch_argmax(const uint16_t *logits, long rows, long V, int32_t *ids, int32_t *tokens, long tok_stride,
                   long tok_cols, const int32_t *step, hipStream_t stream);
 int launch_add_bf16(const uint16_t *a, const uint16_t *b, uint16_t *out, long n, hipStream_t stream);
@@ -321,14 +321,16 @@ static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw,
         if (rc != SC_EUNSUPPORTED) return rc;
     }
     if (band_first(M, N, K, bits)) {
-        // the band kernel's split-K pass applies silu(gate) * up itself
+        // the band kernel's split-K pass applies silu(gate) * up itself (unsplit, the
+        // activation's own launch)
         rc = launch_qgemm_band(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half, 0,
-                               0);
+                               0, nullptr, gu_scratch);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
     if (M > 8 && M <= 32) {
-        // the 9-32-row GEMV's split-K pass applies silu(gate) * up itself
-        rc = launch_qgemv16(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half);
+        // the 9-32-row GEMV, likewise
+        rc = launch_qgemv16(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half, nullptr,
+                            gu_scratch);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
     if (M > 160) {

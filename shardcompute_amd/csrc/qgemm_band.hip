@@ -572,12 +572,15 @@ int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits) {
 // no_alloc: the split-K partials go to the allocation-free scratch array (shapes that
 // need more are SC_EUNSUPPORTED) instead of the library-owned buffer.
 // swiglu_half > 0: the weight is gate|up stacked (N = 2 swiglu_half) and y
-// [M, swiglu_half] receives silu(gate) * up, applied by the split-K pass.
+// [M, swiglu_half] receives silu(gate) * up, applied by the split-K pass.  K in one piece
+// needs no scratch and no fp32 partials: the product goes to gate_up [M, N] (16-byte
+// aligned) and the activation reads it (8B gate|up at 100 and 160 rows TIMES).
 // keep (plain products): the partials are left to the caller's pass (keep->splits > 0)
 // instead of being summed into y.
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
-                      bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep) {
+                      bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep,
+                      uint16_t *gate_up) {
     if (M < 1 || M > 256 || N < 1) return SC_EUNSUPPORTED;
     if (bits != 4 && bits != 8) return SC_EUNSUPPORTED;
     if (K % 512) return SC_EUNSUPPORTED;                 // whole 8-group scale/bias blocks
@@ -597,7 +600,9 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
     a.x = x; a.wq = reinterpret_cast<const uint8_t *>(wq); a.s = s; a.b = b; a.bias = bias; a.y = y;
     a.partials = nullptr;
     a.M = M; a.N = N; a.K = K; a.G = G; a.gps = 8 * bps;
-    const bool with_partials = ksplit > 1 || swiglu_half > 0;
+    const bool then_act = swiglu_half && ksplit == 1 && gate_up && (uintptr_t)y % 16 == 0;
+    const bool with_partials = ksplit > 1 || (swiglu_half && !then_act);
+    if (then_act) a.y = gate_up;
     if (with_partials) {
         const size_t need = (size_t)ksplit * M * N;
         if (no_alloc) {
@@ -626,6 +631,7 @@ int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, 
                      : launch_band_mt<8, 8>(a, nw, tiles, ksplit, stream);
     }
     if (rc) return rc;
+    if (then_act) return launch_silu_mul(gate_up, M, swiglu_half, y, stream);
     if (keep) {
         keep->partials = with_partials ? a.partials : nullptr;
         keep->splits = with_partials ? ksplit : 0;

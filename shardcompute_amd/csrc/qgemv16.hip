@@ -484,12 +484,13 @@ static int launch_gemv16_t(const Gemv16Args &a, const Gemv16Plan &p, hipStream_t
 // no_alloc: the split-K partials go to the file-scope scratch array (shapes that
 // need more than it holds are rejected) instead of the library-owned buffer.
 // swiglu_half > 0: the weight is gate|up stacked (N = 2 swiglu_half) and y [M, swiglu_half]
-// receives silu(gate) * up, applied by the partials' pass (which then always runs).
+// receives silu(gate) * up, applied by the partials' pass; K in one piece needs no scratch:
+// the product goes to gate_up [M, N] (16-byte aligned) and the activation reads it.
 // keep (plain products): the partials are left to the caller's pass (keep->splits > 0)
 // instead of being summed into y.
 int launch_qgemv16(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b, const uint16_t *bias,
                    uint16_t *y, int M, int N, int K, int bits, hipStream_t stream, bool no_alloc, int swiglu_half,
-                   SplitKeep *keep) {
+                   SplitKeep *keep, uint16_t *gate_up) {
     if (M < 1 || M > 32) return SC_EUNSUPPORTED;
     if (swiglu_half && (swiglu_half < 0 || N != 2 * swiglu_half)) return SC_EUNSUPPORTED;
     if (((uintptr_t)s % 16) || ((uintptr_t)b % 16)) return SC_EUNSUPPORTED;
@@ -500,7 +501,9 @@ int launch_qgemv16(const uint16_t *x, const uint32_t *wq, const uint16_t *s, con
     a.x = x; a.wq = wq; a.s = s; a.b = b; a.bias = bias; a.y = y; a.partials = nullptr;
     a.M = M; a.N = N; a.K = K; a.G = K / 64; a.spans_per_split = p.spans_per_split;
     a.tiles_per_wg = p.tiles_per_wg;
-    const bool with_partials = p.splits > 1 || swiglu_half > 0;
+    const bool then_act = swiglu_half && p.splits == 1 && gate_up && (uintptr_t)y % 16 == 0;
+    const bool with_partials = p.splits > 1 || (swiglu_half && !then_act);
+    if (then_act) a.y = gate_up;
     if (with_partials) {
         const size_t need = (size_t)p.splits * M * N;
         if (no_alloc) {
@@ -526,6 +529,7 @@ int launch_qgemv16(const uint16_t *x, const uint32_t *wq, const uint16_t *s, con
     return set_error(SC_EUNSUPPORTED, "qgemv16: bits=%d", bits);
 #undef SC_G16
     if (rc) return rc;
+    if (then_act) return launch_silu_mul(gate_up, M, swiglu_half, y, stream);
     if (keep) {
         keep->partials = with_partials ? a.partials : nullptr;
         keep->splits = with_partials ? p.splits : 0;

@@ -270,6 +270,8 @@ struct SplitKeep {
 // receives silu(gate) * up of the rounded values.
 int launch_qmm_finalize(const float *partials, int splits, int M, int N, const uint16_t *bias, uint16_t *y, int half,
                         hipStream_t stream);
+// out [rows, I] = silu(gate) * up of gu [rows, 2 I] (decode.hip); gu and out 16-byte aligned
+int launch_silu_mul(const uint16_t *gu, long rows, long I, uint16_t *out, hipStream_t stream);
 
 // Arg-max key of a bf16 value: the order-preserving 16-bit image of the value
 // (NaN above +inf, -0.0 equal to +0.0) over ~index, so the larger key is the larger

@@ -448,17 +448,17 @@ def qmm_swiglu(x, wq, scales, biases, norm_weight=None, eps=1e-5, residual=None,
         raise ValueError("a residual needs the norm weight")
     if residual is not None:
         _rows(residual, K, "residual")
-    act = act_out if act_out is not None else torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
-    _rows(act, I, "act_out")
-    gu = gate_up_scratch if gate_up_scratch is not None else torch.empty((M, N), dtype=torch.bfloat16,
-                                                                          device=x.device)
-    _rows(gu, N, "gate_up_scratch")
+    act = x.new_empty((M, I)) if act_out is None else _rows(act_out, I, "act_out")
+    gu = x.new_empty((M, N)) if gate_up_scratch is None else _rows(gate_up_scratch, N, "gate_up_scratch")
     ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
     rc = lib.sc_qmm_swiglu_bf16_ws(_ptr(x), _ptr(residual), _ptr(norm_weight), float(eps), _ptr(h_out), _ptr(xn),
                                    _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(act), _ptr(gu), M, I, K,
                                    bits, group_size, _ptr(ws), ws_bytes, _stream(x))
-    _check(rc, "sc_qmm_swiglu_bf16")
-    return act.reshape(*lead, I), (xn.reshape(*lead, K) if xn is not None else None)
+    if rc:
+        _check(rc, "sc_qmm_swiglu_bf16")
+    if act_out is not None or len(lead) != 1:
+        act = act.reshape(*lead, I)
+    return act, (xn.reshape(*lead, K) if xn is not None else None)
 
 
 def vocab_gather(ids, table, vocab_start=0, out=None):

@@ -113,7 +113,7 @@ class FusedColumns:
         writes the gated activation directly.  Returns act."""
         if not self._current():
             self.build()
-        if len(self.parts) != 2 or self.widths[0] != self.widths[1]:
+        if len(self.parts) != 2 or self.parts[0].local_out_features != self.parts[1].local_out_features:
             raise ValueError("swiglu needs a gate|up pair of equal widths")
         if norm is not None:
             norm._check()

@@ -87,11 +87,13 @@ class ParallelMLP:
 
     def intermediate(self, x2, gu_out=None, out=None):
         """f(gate(x)) * up(x) (gated) or f(up(x)) for x2 ``[rows, hidden]`` ->
-        ``[rows, local_intermediate]``."""
-        if self.fused_swiglu and x2.dtype == torch.bfloat16 and x2.shape[0] > 0:
-            # silu(gate) * up inside the gate|up product: the same bits as the product
-            # followed by the activation, without writing and reading [rows, 2 I]
-            return self.gate_up.swiglu_call(x2.contiguous(), None, act_out=out, gu_out=gu_out)
+        ``[rows, local_intermediate]``, into ``out`` where given; ``gu_out`` receives the
+        gate|up product (gated)."""
+        if self.fused_swiglu and gu_out is None and out is None and x2.dtype == torch.bfloat16 and x2.numel() > 0:
+            # silu(gate) * up inside the gate|up product, without writing and reading
+            # [rows, 2 I].  From 9 rows on the same bits as the product followed by the
+            # activation; up to 8 rows the fp32 sums run in another order.
+            return self.gate_up.swiglu_call(x2.contiguous())
         if self.use_gated:
             gu = self.gate_up(x2, out=gu_out)
             return _lib.act(gu, self.activation_name, gated=True, out=out)

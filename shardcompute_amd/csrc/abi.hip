@@ -31,7 +31,6 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
 int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                      const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                      int swiglu_half, bool no_alloc);
-int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits);
 int launch_qgemm_band(const uint16_t *x, const uint32_t *wq, const uint16_t *s, const uint16_t *b,
                       const uint16_t *bias, uint16_t *y, int M, int N, int K, int bits, hipStream_t stream,
                       bool no_alloc, int swiglu_half, int force_nw, int force_split, SplitKeep *keep = nullptr,
@@ -174,26 +173,20 @@ static int check_qmm(const void *x, const void *wq, const void *s, const void *b
 // kernels compute 32 rows and the band's stream is the faster (8B gate|up at 20, 24
 // and 32 rows 28, 31, 30 against 32, 34, 34 us on the GEMV; the 8B lm_head at 32 rows
 // 99 against 119 us); 9-16 rows where the 16-column GEMV's K splits or x staging cost
-// more than the band's stream: K above 4096, up to 8192 weight rows, or up to 16384 at
-// 4 bits and 65536 at 8 (TinyLlama gate|up at 16 rows 11.5 against 12.0 us, W8 12.2 against
-// 15.0; 8B gate|up W8 34.0 against 38.5, W4 24.6 against 24.4; the 8B lm_head 77 against 70,
-// W8 139 against 135).  Above 8192 rows of K up to 4096 only where the scratch is needed no
-// more than on the GEMV: the band's partials fit the allocation-free array, so that
-// sc_qmm_bf16_noalloc stays bit-equal, and the GEMV would split K as well (it does below
-// 8 tiles of 16 rows a CU; from there on it needs no scratch);
+// more than the band's stream: K above 4096 or at most 8192 weight rows (8B down at 16
+// rows 16 against 25 us).  Wider products of 9-16 rows are a matter of rounds: where the
+// band's tiles times splits just miss one (W8 24560 x 3072) 33 against 22 us on the GEMV,
+// where they fill it (W8 11264 x 2048) 12 against 15; of 150 sizes a third lost, most of
+// the others tied, so they stay on the GEMV;
 // and 8 rows with K of 4096 or more (8B q|k|v, gate|up, down 10, 24, 16 against 13,
 // 25, 26 us on the 8-row GEMV; K = 2048 is a tie).  4-7 rows, and 8 rows of a smaller K, are
 // up to 1.6 times faster here too (8B down at 4 rows 16 against 25 us), but stay on the GEMV:
 // it needs no split-K scratch, so those products may run on several streams at once and
 // be a process's first call under capture.
-static bool band_first(int64_t M, int64_t N, int64_t K, int bits) {
+static bool band_first(int64_t M, int64_t N, int64_t K) {
     if (M > 32) return M <= 160;
     if (M == 8) return K >= 4096;
-    if (M > 16 || (M > 8 && (K > 4096 || N <= 8192))) return true;
-    if (M <= 8 || N > (bits == 4 ? 16384 : 65536) || K % 512) return false;
-    const int64_t partials = qgemm_band_partials(M, N, K, bits);
-    return partials * (int64_t)sizeof(float) <= (int64_t)SC_QMM_NOALLOC_SCRATCH_BYTES &&
-           (!partials || (N + 15) / 16 < 8 * (int64_t)device_info().num_cus);
+    return M > 16 || (M > 8 && (K > 4096 || N <= 8192));
 }
 
 // The caller's workspace of a call (none: ws null), for the products whose weights are
@@ -218,8 +211,8 @@ static int qmm_dispatch(const uint16_t *x, const uint32_t *wq, const uint16_t *s
         rc = launch_qgemm_mid(x, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, 0, no_alloc);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
-    if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K, bits) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
-                                                                                    : SC_QMM_PATH_GEMM;
+    if (path == SC_QMM_PATH_AUTO) path = band_first(M, N, K) ? SC_QMM_PATH_BAND : M <= 32 ? SC_QMM_PATH_GEMV
+                                                                              : SC_QMM_PATH_GEMM;
     if (path == SC_QMM_PATH_BAND) {
         // any M <= 256: the weight-streaming band kernel; shapes it does not take (K not
         // a multiple of 512, partials beyond the no-alloc scratch) go to the GEMVs up to
@@ -320,7 +313,7 @@ static int qmm_fused(const uint16_t *x, const uint16_t *res, const uint16_t *nw,
                                 wsp.bytes);
         if (rc != SC_EUNSUPPORTED) return rc;
     }
-    if (band_first(M, N, K, bits)) {
+    if (band_first(M, N, K)) {
         // the band kernel's split-K pass applies silu(gate) * up itself (unsplit, the
         // activation's own launch)
         rc = launch_qgemm_band(xin, wq, s, b, bias, y, (int)M, (int)N, (int)K, bits, st, false, (int)swiglu_half, 0,

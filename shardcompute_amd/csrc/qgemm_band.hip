@@ -561,12 +561,6 @@ static BandPlan plan_band(int M, int N, int K, int bits, int force_nw, int force
     return p;
 }
 
-// Floats of split-K partials that a product on this kernel takes from the scratch (0: none).
-int64_t qgemm_band_partials(int64_t M, int64_t N, int64_t K, int bits) {
-    const BandPlan p = plan_band((int)M, (int)N, (int)K, bits, 0, 0);
-    return p.ksplit > 1 ? p.ksplit * M * N : 0;
-}
-
 // Returns SC_EUNSUPPORTED when the shape does not suit this kernel (the caller falls
 // back).  force_nw / force_split (0 = automatic) pin the plan for measurements.
 // no_alloc: the split-K partials go to the allocation-free scratch array (shapes that

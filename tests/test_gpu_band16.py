@@ -41,12 +41,12 @@ def test_band_up_to_16_rows(device, bits, M):
 
 
 @pytest.mark.parametrize("bits,M,N,K", [
-    (4, 16, 8192, 1024), (4, 16, 11264, 2048), (4, 16, 14000, 4096), (4, 9, 16384, 512),  # fit / fit / exceed / unsplit
+    (4, 16, 8192, 1024), (4, 16, 11264, 2048), (4, 16, 14000, 4096), (4, 9, 16384, 512),  # the band's would: fit / fit / exceed / be none
     (8, 16, 32752, 1024), (8, 9, 32768, 1024), (8, 16, 22000, 4096), (8, 9, 43528, 1024)])
 def test_wide_products_of_9_to_16_rows_need_no_more_scratch(device, bits, M, N, K):
-    """The allocation-free entry gives sc_qmm_bf16's bits on either side of every line of
-    the 9-16-row rule (8192, 16384 and 65536 weight rows, the partials' limit, the sizes
-    that the GEMV does not split)."""
+    """The allocation-free entry gives sc_qmm_bf16's bits on either side of the 9-16-row rule's
+    line (8192 weight rows) and for wider products, whose partials on the band kernel would
+    exceed its scratch or be scratch that the GEMV, unsplit, does not take."""
     rng = np.random.default_rng(N + K)
     x = dev_bf16(f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32)))
     per = 8 if bits == 4 else 4
@@ -63,3 +63,16 @@ def test_wide_products_of_9_to_16_rows_need_no_more_scratch(device, bits, M, N, 
     got = bf16_to_f32(host_u16(y)).astype(np.float64)[:, cols]
     _, e = np.frexp(np.abs(ref))
     assert np.all(np.abs(got - ref) <= 2 * np.ldexp(1.0, e - 8) + 1e-5 * np.max(np.abs(ref)))
+
+
+@pytest.mark.parametrize("bits,M,N,K", [(8, 11, 24560, 3072), (8, 9, 44752, 4096), (4, 13, 14648, 3072)])
+def test_wide_products_of_9_to_16_rows_run_on_the_gemv(device, bits, M, N, K):
+    """The band kernel's tiles and splits miss one round of the CUs here by a little (1.1-1.5
+    times the GEMV's time); its sums run in another order, so the bits tell the two apart."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    x = torch.randn((M, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = _lib.quantize(torch.randn((N, K), generator=g, device="cuda").mul_(0.02), bits=bits)
+    y, yg, yb = (_lib.qmm(x, *w, bits=bits, path=p) for p in (_lib.PATH_AUTO, _lib.PATH_GEMV, _lib.PATH_BAND))
+    assert not torch.equal(yg, yb)
+    assert torch.equal(y, yg)

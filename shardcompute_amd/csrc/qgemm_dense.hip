@@ -66,7 +66,6 @@ struct DenseArgs {
     int64_t ldy;              // y's row stride
     int n_base;               // column of y (SwiGLU: of the product) that column 0 of w stands for
     int swiglu_i;             // I > 0: columns 2j, 2j + 1 are gate j and up j; y receives act [M, I]
-    int vec;                  // rows of y are aligned for 16-byte (SwiGLU: 8-byte) stores
     int mt, nt, tiles;
     int group_m;              // row tiles a run of tiles walks before the next column
 };
@@ -269,34 +268,33 @@ qgemm_dense_kernel(DenseArgs a) {
 
     // ---- epilogue: acc[i][2 p] and acc[i][2 p + 1] of lane (li, lq) are row
     // m0 + wm WM + 16 i + li, columns n0 + wn WN + 32 p + 8 lq .. + 7, rounded to bf16, the
-    // bias added and rounded again.  FAST: a tile inside the matrix, aligned rows, no bias.
-    auto store = [&](auto fast_tag, auto swiglu_tag) __attribute__((always_inline)) {
-        constexpr bool FAST = decltype(fast_tag)::value != 0, SWIGLU = decltype(swiglu_tag)::value != 0;
+    // bias added and rounded again
+    auto store = [&](auto swiglu_tag) __attribute__((always_inline)) {
+        constexpr bool SWIGLU = decltype(swiglu_tag)::value != 0;
+        const int nl = n0 + wn * WN + 8 * lq;
+        uint32_t bb[NJ / 2][4] = {};
+        if (a.bias) {
+#pragma unroll
+            for (int p = 0; p < NJ / 2; ++p)
+                load_bias8<SWIGLU>(bb[p], a.bias, a.n_base + nl + 32 * p, nl + 32 * p, N, a.swiglu_i);
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int m = m0 + wm * WM + 16 * i + li;
-            if (!FAST && m >= M) continue;
+            if (m >= M) continue;
             uint16_t *yr = a.y + (size_t)m * a.ldy;
 #pragma unroll
             for (int p = 0; p < NJ / 2; ++p) {
-                const int n = n0 + wn * WN + 32 * p + 8 * lq;
-                const int c = a.n_base + n;                       // product column
                 uint32_t o[4] = {cvt_pk_bf16(acc[i][2 * p][0], acc[i][2 * p][1]),
                                  cvt_pk_bf16(acc[i][2 * p][2], acc[i][2 * p][3]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][0], acc[i][2 * p + 1][1]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][2], acc[i][2 * p + 1][3])};
-                store_cols8<FAST, SWIGLU>(o, yr, c, n, N, a.bias, a.swiglu_i);
+                store_cols8<SWIGLU>(o, yr, a.n_base + nl + 32 * p, nl + 32 * p, N, a.bias != nullptr, bb[p]);
             }
         }
     };
-    const bool fast = a.vec && !a.bias && m0 + BM <= M && n0 + BN <= N;
-    if (a.swiglu_i) {
-        if (fast) store(int_c<1>{}, int_c<1>{});
-        else store(int_c<0>{}, int_c<1>{});
-    } else {
-        if (fast) store(int_c<1>{}, int_c<0>{});
-        else store(int_c<0>{}, int_c<0>{});
-    }
+    if (a.swiglu_i) store(int_c<1>{});
+    else store(int_c<0>{});
 }
 
 // Rows [r0, r0 + rows) of the product's weights as bf16 [rows, K].  half = I > 0: product
@@ -397,7 +395,7 @@ static int launch_dense(const DenseArgs &a, hipStream_t stream) {
 // 103 -> 93, 3072 x 2048 x 5632 90 -> 89, 3072 x 8192 x 1024 67 -> 66, 2048 x 8192 x 1024
 // 42 -> 43, 4096 x 2560 x 2048 56 -> 51, 3072 x 2560 x 2048 40 -> 43.
 int64_t qgemm_dense_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M < 1024 || M > (1 << 30) || N < 256 || N > (1 << 30) || K < 1024 || K > (1 << 20) || K % BK) return 0;
+    if (M < 1024 || M > (1 << 30) || N < 256 || N > (1 << 30) || K < 1024 || K > (1 << 20) || K % BK || N % 8) return 0;
     if (M * N < (K < 2048 ? 20000000 : M < 1280 ? 11500000 : 1 << 23)) return 0;
     const int64_t row = K * 2;
     int64_t rows = N;
@@ -412,6 +410,7 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
     const int64_t need = qgemm_dense_workspace_bytes(M, N, K);
     if (need == 0 || !ws || ws_bytes < need || ((uintptr_t)ws % 16) != 0) return SC_EUNSUPPORTED;
     if ((bits != 4 && bits != 8) || (swiglu_half && N != 2 * swiglu_half)) return SC_EUNSUPPORTED;
+    if (!wide_rows(y, N, swiglu_half)) return SC_EUNSUPPORTED;
     if (device_info().max_lds_per_block < 2 * (BM + 256) * ROW_BYTES) return SC_EUNSUPPORTED;
     const int rows = (int)(need / ((int64_t)K * 2));
     DenseArgs a;
@@ -419,7 +418,6 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
     a.M = M; a.K = K;
     a.ldy = swiglu_half ? swiglu_half : N;
     a.swiglu_i = swiglu_half;
-    a.vec = swiglu_half ? (swiglu_half % 4 == 0 && (uintptr_t)y % 8 == 0) : (N % 8 == 0 && (uintptr_t)y % 16 == 0);
     a.mt = (M + BM - 1) / BM;
     a.nt = a.tiles = 0;
     for (int n0 = 0; n0 < N; n0 += rows) {

@@ -65,7 +65,6 @@ struct MidArgs {
     int gps;                  // groups per K split, a multiple of 8
     int64_t ldy;
     int swiglu_i;             // I > 0: product columns 2j, 2j + 1 are weight rows j and I + j
-    int vec;
     int mt, nt, tiles;
 };
 
@@ -221,37 +220,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int m = m0 + 16 * i + li;
             if (m >= M) continue;
             float *p = pz + (size_t)m * N + n;
-            if (N % 4 == 0 && n + 8 <= N) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    *reinterpret_cast<float4 *>(p + 4 * j) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (n + e < N) p[e] = acc[i][e >> 2][e & 3];
-            }
+            for (int j = 0; j < 2; ++j)
+                *reinterpret_cast<float4 *>(p + 4 * j) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
         }
         return;
     }
-    auto store = [&](auto fast_tag, auto swiglu_tag) __attribute__((always_inline)) {
-        constexpr bool FAST = decltype(fast_tag)::value, SWIGLU = decltype(swiglu_tag)::value;
+    auto store = [&](auto swiglu_tag) __attribute__((always_inline)) {
+        constexpr bool SWIGLU = decltype(swiglu_tag)::value;
+        uint32_t bb[4] = {};
+        if (a.bias) load_bias8<SWIGLU>(bb, a.bias, n, n, N, a.swiglu_i);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int m = m0 + 16 * i + li;
             if (m >= M) continue;
             uint32_t o[4] = {cvt_pk_bf16(acc[i][0][0], acc[i][0][1]), cvt_pk_bf16(acc[i][0][2], acc[i][0][3]),
                              cvt_pk_bf16(acc[i][1][0], acc[i][1][1]), cvt_pk_bf16(acc[i][1][2], acc[i][1][3])};
-            store_cols8<FAST, SWIGLU>(o, a.y + (size_t)m * a.ldy, n, n, N, a.bias, a.swiglu_i);
+            store_cols8<SWIGLU>(o, a.y + (size_t)m * a.ldy, n, n, N, a.bias != nullptr, bb);
         }
     };
-    const bool fast = a.vec && !a.bias && n0 + NB <= N;
-    if (a.swiglu_i) {
-        if (fast) store(std::true_type{}, std::true_type{});
-        else store(std::false_type{}, std::true_type{});
-    } else {
-        if (fast) store(std::true_type{}, std::false_type{});
-        else store(std::false_type{}, std::false_type{});
-    }
+    if (a.swiglu_i) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 template <int BITS>
@@ -287,6 +276,7 @@ int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, c
                      int swiglu_half, bool no_alloc) {
     if (K % 512 || M < 1 || N < 1 || (int64_t)K > (1 << 20)) return SC_EUNSUPPORTED;
     if ((bits != 4 && bits != 8) || (swiglu_half && N != 2 * swiglu_half)) return SC_EUNSUPPORTED;
+    if (!wide_rows(y, N, swiglu_half)) return SC_EUNSUPPORTED;
     if (((uintptr_t)x | (uintptr_t)wq | (uintptr_t)s | (uintptr_t)b) % 16) return SC_EUNSUPPORTED;
     if (device_info().max_lds_per_block < MidGeo<8>::LDS) return SC_EUNSUPPORTED;
     MidArgs a;
@@ -295,7 +285,6 @@ int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, c
     a.M = M; a.N = N; a.K = K; a.G = K / 64; a.gps = a.G;
     a.ldy = swiglu_half ? swiglu_half : N;
     a.swiglu_i = swiglu_half;
-    a.vec = swiglu_half ? (swiglu_half % 4 == 0 && (uintptr_t)y % 8 == 0) : (N % 8 == 0 && (uintptr_t)y % 16 == 0);
     a.mt = (M + MB - 1) / MB;
     a.nt = (N + NB - 1) / NB;
     const int64_t tiles = (int64_t)a.mt * a.nt;

@@ -28,10 +28,9 @@ def _inputs(M, N, K, bits, seed):
     return x, wq, s, b, bias, ref, acc
 
 
-# rows and widths at the edges of the 256 x 256 and 256 x 128 tiles, odd widths (element
-# stores), stages of odd number, a last partial round as narrow tiles (12 x 43 wide tiles),
+# rows and widths at the edges of the 256 x 256 and 256 x 128 tiles, stages of odd number, a last partial round as narrow tiles (12 x 43 wide tiles),
 # weights in two column chunks (N K above 2^27), the smallest products taken
-SHAPES = [(1280, 6592, 1088, 4), (1281, 15873, 1024 + 576, 8), (2048, 4096, 4096, 4), (2049, 4104, 2048, 8),
+SHAPES = [(1280, 6592, 1088, 4), (1281, 15880, 1024 + 576, 8), (2048, 4096, 4096, 4), (2049, 4104, 2048, 8),
           (2815, 11008, 2112, 4), (1030, 34000, 4096, 8), (40000, 512, 1024, 4)]
 
 
@@ -62,8 +61,8 @@ def test_dense_swiglu_equals_product_then_gate(device, M, I, K, bits, with_bias)
 
 
 def test_workspace_forms(device):
-    """A misaligned output takes element stores, a small, null or misaligned workspace the
-    fused GEMM; every form agrees with the reference."""
+    """A misaligned output and a small, null or misaligned workspace take the fused GEMM; every
+    form agrees with the reference."""
     M, N, K, bits = 2048, 4096, 1024 * 2, 4
     x, wq, s, b, _, ref, acc = _inputs(M, N, K, bits, 7)
     lib, P = _lib.load(), ctypes.c_void_p
@@ -81,6 +80,16 @@ def test_workspace_forms(device):
         assert rc == 0, lib.sc_last_error()
         bad = (y.view(M, N).double() - ref).abs() > 2.0 ** -8 * ref.abs() + acc
         assert not bad.any(), (y_off, ws_off, ws_bytes)
+
+
+def test_rows_of_element_stores_take_the_fused_gemm(device):
+    """Widths that are no multiple of 8 want no workspace (2-byte stores cost the dense kernel
+    more than it gains on most of them) and give the fused GEMM's bits."""
+    M, N, K, bits = 1300, 16001, 1088, 4
+    assert _lib.load().sc_qmm_workspace_bytes(M, N, K) == 0 < _lib.load().sc_qmm_workspace_bytes(M, N - 1, K)
+    x, wq, s, b, bias, _, _ = _inputs(M, N, K, bits, 3)
+    assert torch.equal(_lib.qmm(x, wq, s, b, bias=bias, bits=bits),
+                       _lib.qmm(x, wq, s, b, bias=bias, bits=bits, path=_lib.PATH_GEMM))
 
 
 def test_dense_under_graph_capture(device):

@@ -19,10 +19,10 @@ def _inputs(M, N, K, bits):
     return x, wq, s, b, torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
 
 
-# one row and one column past a tile, ragged and odd widths, one scale block, the largest tile
+# one row and one column past a tile, ragged widths and odd ones (which run on the fused GEMM), one scale block, the largest tile
 # count and one past it, K split with and without enough blocks for its splits
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,N,K", [(161, 128, 512), (257, 129, 1024), (300, 1001, 512), (170, 77, 2048),
+@pytest.mark.parametrize("M,N,K", [(161, 128, 512), (257, 129, 1024), (300, 1001, 512), (170, 77, 2048), (170, 1000, 1024), (201, 72, 5120),
                                    (2048, 2048, 512), (2049, 2048, 512), (333, 2048, 5632), (200, 300, 4096)])
 def test_mid_against_reference(device, M, N, K, bits):
     print(f"mid M={M} N={N} K={K} W{bits}", flush=True)

@@ -18,12 +18,12 @@ __device__ __forceinline__ void load_bias8(uint32_t (&bb)[4], const uint16_t *bi
 // o: the lane's columns rounded to bf16; yr: the output row.  The bias, if there is one, is
 // added to the rounded values and rounded again.  SWIGLU: the row receives silu(gate) * up.
 // N is a multiple of 8, so the columns lie all inside the matrix or all outside, and rows are
-// aligned for 16-byte (SwiGLU: 8-byte) stores.
-template <bool SWIGLU>
+// aligned for 16-byte (SwiGLU: 8-byte) stores.  INNER: all inside, no bias.
+template <bool INNER, bool SWIGLU>
 __device__ __forceinline__ void store_cols8(uint32_t (&o)[4], uint16_t *yr, int c, int n, int N, bool has_bias,
                                             const uint32_t (&bb)[4]) {
-    if (n >= N) return;
-    if (has_bias) {
+    if (!INNER && n >= N) return;
+    if (!INNER && has_bias) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             o[e] = cvt_pk_bf16(bf2f(o[e] & 0xFFFFu) + bf2f(bb[e] & 0xFFFFu), bf2f(o[e] >> 16) + bf2f(bb[e] >> 16));

@@ -12,9 +12,9 @@
 // the stage loop holds MFMAs, LDS reads and LDS-DMA only.  The dequantization costs
 // N K (2 + bits/8) bytes of traffic once, which pays from 1000-2000 rows (the rule at
 // qgemm_dense_workspace_bytes).  Measured with the dequantization (medians on one box,
-// qgemm.hip -> here, W4): 2048 x 28672 x 4096 482 -> 418 us (1150 TFLOP/s), 2048 x 4096 x
-// 14336 250 -> 230, 2048 x 7168 x 8192 237 -> 190 (1269), 4096 x 28672 x 4096 935 -> 733
-// (1313), 8192 x 4096 x 4096 265 -> 196 (1404); W8 8192 x 7168 x 8192 996 -> 713 (1350).
+// qgemm.hip -> here, W4): 2048 x 28672 x 4096 480 -> 413 us (1166 TFLOP/s), 2048 x 4096 x
+// 14336 247 -> 222, 2048 x 6144 x 4096 109 -> 88 (1169), ragged 3821 x 15904 x 8384 964 -> 801
+// (1272), 8192 x 7168 x 8192 902 -> 678 (1419); W8 8192 x 7168 x 8192 957 -> 685 (1404).
 //
 // qgemm_dense_kernel:
 // * Workgroup tile 256 x 256 on 4 waves (one per SIMD, each 128 x 128, its 256
@@ -269,11 +269,12 @@ qgemm_dense_kernel(DenseArgs a) {
     // ---- epilogue: acc[i][2 p] and acc[i][2 p + 1] of lane (li, lq) are row
     // m0 + wm WM + 16 i + li, columns n0 + wn WN + 32 p + 8 lq .. + 7, rounded to bf16, the
     // bias added and rounded again
-    auto store = [&](auto swiglu_tag) __attribute__((always_inline)) {
-        constexpr bool SWIGLU = decltype(swiglu_tag)::value != 0;
+    // INNER: a tile inside the matrix, no bias (predicates for all cost 0.5 % of a product)
+    auto store = [&](auto inner_tag, auto swiglu_tag) __attribute__((always_inline)) {
+        constexpr bool INNER = decltype(inner_tag)::value != 0, SWIGLU = decltype(swiglu_tag)::value != 0;
         const int nl = n0 + wn * WN + 8 * lq;
         uint32_t bb[NJ / 2][4] = {};
-        if (a.bias) {
+        if (!INNER && a.bias) {
 #pragma unroll
             for (int p = 0; p < NJ / 2; ++p)
                 load_bias8<SWIGLU>(bb[p], a.bias, a.n_base + nl + 32 * p, nl + 32 * p, N, a.swiglu_i);
@@ -281,7 +282,7 @@ qgemm_dense_kernel(DenseArgs a) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int m = m0 + wm * WM + 16 * i + li;
-            if (m >= M) continue;
+            if (!INNER && m >= M) continue;
             uint16_t *yr = a.y + (size_t)m * a.ldy;
 #pragma unroll
             for (int p = 0; p < NJ / 2; ++p) {
@@ -289,12 +290,18 @@ qgemm_dense_kernel(DenseArgs a) {
                                  cvt_pk_bf16(acc[i][2 * p][2], acc[i][2 * p][3]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][0], acc[i][2 * p + 1][1]),
                                  cvt_pk_bf16(acc[i][2 * p + 1][2], acc[i][2 * p + 1][3])};
-                store_cols8<SWIGLU>(o, yr, a.n_base + nl + 32 * p, nl + 32 * p, N, a.bias != nullptr, bb[p]);
+                store_cols8<INNER, SWIGLU>(o, yr, a.n_base + nl + 32 * p, nl + 32 * p, N, a.bias != nullptr, bb[p]);
             }
         }
     };
-    if (a.swiglu_i) store(int_c<1>{});
-    else store(int_c<0>{});
+    const bool inner = !a.bias && m0 + BM <= M && n0 + BN <= N;
+    if (a.swiglu_i) {
+        if (inner) store(int_c<1>{}, int_c<1>{});
+        else store(int_c<0>{}, int_c<1>{});
+    } else {
+        if (inner) store(int_c<1>{}, int_c<0>{});
+        else store(int_c<0>{}, int_c<0>{});
+    }
 }
 
 // Rows [r0, r0 + rows) of the product's weights as bf16 [rows, K].  half = I > 0: product
@@ -364,39 +371,60 @@ static int launch_dense_cols(const DenseArgs &full, int n0, int nc, hipStream_t 
     return SC_OK;
 }
 
-static int launch_dense(const DenseArgs &a, hipStream_t stream) {
-    // The tile width with the shorter estimate of rounds x tile time (a 256 x 128 tile
-    // takes 0.64 of a 256 x 256 one), and a partial last round of wide tiles that fills at
-    // most half the CUs as narrow tiles: the rules of qgemm.hip, whose ratio holds here
-    // (M = 2048, K = 4096: 61 us a round of narrow tiles, 95 us of wide ones).
+// The columns [0, wide) of a launch of mt row tiles run as 256 x 256 tiles, the others as
+// 256 x 128 ones; cost: the estimate in hundredths of a round of wide tiles.
+struct DensePlan {
+    int wide;
+    int64_t cost;
+};
+
+// Wide tiles, narrow ones, or whole rounds of wide ones and the last columns narrow: the
+// shortest estimate of rounds x tile time, a 256 x 128 tile taking 0.7 of a 256 x 256 one (one
+// round at M = 2048, K 2048, 4096, 8192: narrow 37, 68, 122 us, wide 53, 94, 176).  Measured
+// against the rule before, 0.64 and a mixed launch only where the last round splits evenly
+// (W4): 1.5 rounds, mixed, 3031 x 7680 x 3968 185 -> 162 us; 2 wide rounds where 3 narrow
+// ones ran, 1680 x 13760 x 7808 453 -> 371.
+static DensePlan plan_dense(int mt, int64_t cols) {
     const int cus = device_info().num_cus;
-    const int64_t tiles256 = (int64_t)a.mt * ((a.N + 255) / 256);
-    const int64_t waves256 = (tiles256 + cus - 1) / cus;
-    const int64_t waves128 = ((int64_t)a.mt * ((a.N + 127) / 128) + cus - 1) / cus;
-    if (100 * waves256 > 64 * waves128) return launch_dense_cols<128, 4, 2>(a, 0, a.N, stream);
-    const int64_t r = tiles256 % cus;
-    if (r > 0 && tiles256 > cus && a.N % 256 == 0 && r % a.mt == 0 && 2 * r <= cus) {
-        const int n1 = a.N - (int)(r / a.mt) * 256;
-        const int rc = launch_dense_cols<256, 2, 2>(a, 0, n1, stream);
-        if (rc) return rc;
-        return launch_dense_cols<128, 4, 2>(a, n1, a.N - n1, stream);
+    const auto rounds = [&](int64_t n, int bn) { return ((int64_t)mt * ((n + bn - 1) / bn) + cus - 1) / cus; };
+    DensePlan best{(int)cols, 100 * rounds(cols, 256)};
+    const int64_t full = (int64_t)mt * ((cols + 255) / 256) / cus;      // whole rounds of wide tiles,
+    const int64_t n1 = full * cus / mt * 256;                           // the columns they hold
+    for (const int64_t w : {(int64_t)0, n1}) {
+        if (w >= cols) continue;
+        const int64_t cost = (w ? 100 * full : 0) + 70 * rounds(cols - w, 128);
+        if (cost < best.cost) best = DensePlan{(int)w, cost};
     }
-    return launch_dense_cols<256, 2, 2>(a, 0, a.N, stream);
+    return best;
+}
+
+static int launch_dense(const DenseArgs &a, hipStream_t stream) {
+    const int w = plan_dense(a.mt, a.N).wide;
+    if (w > 0) {
+        const int rc = launch_dense_cols<256, 2, 2>(a, 0, w, stream);
+        if (rc || w == a.N) return rc;
+    }
+    return launch_dense_cols<128, 4, 2>(a, w, a.N - w, stream);
 }
 
 // Bytes of workspace the dense path wants for a product, 0 where the fused GEMM is the
 // faster (or the shape is not taken).  The dequantization's cost is per weight and two
 // launches, the gain per product element, and a dense tile is slower to start and end, so
 // the line is drawn at 2^23 outputs (128 wide tiles, half the CUs), 1280 rows; from 1024
-// rows at 11.5 M outputs; and with K below 2048, where start and end weigh more, 20 M.
+// rows at 11.5 M outputs, K up to 8192 (above, the dequantization is a sixth of the time and
+// the two tie: 1057 x 12544 x 11072 340 -> 348, 1143 x 18672 x 10752 537 -> 525); and with K
+// below 2048, where start and end weigh more, 20 M, below 1536 26 M.
 // Measured at the line, fused GEMM -> here, W4 (W8), us: 2048 x 4096 x 4096 77 -> 72
 // (78 -> 71), 1536 x 4096 x 4096 65 -> 67, 1280 x 8192 x 3584 96 -> 86, 1024 x 8192 x 3584
 // 70 -> 70 (69 -> 71), 1024 x 11264 x 2048 63 -> 62 (65 -> 58), 4096 x 2048 x 5632
-// 103 -> 93, 3072 x 2048 x 5632 90 -> 89, 3072 x 8192 x 1024 67 -> 66, 2048 x 8192 x 1024
-// 42 -> 43, 4096 x 2560 x 2048 56 -> 51, 3072 x 2560 x 2048 40 -> 43.
+// 103 -> 93, 3072 x 2048 x 5632 90 -> 89, 3178 x 8448 x 1024 71 -> 65, 6144 x 4096 x 1024
+// 60 -> 62, 1024 x 22528 x 1280 69 -> 71, 4096 x 2560 x 2048 56 -> 51, 3072 x 2560 x 2048
+// 40 -> 43.  Over 900 sizes above the line 1.21 times as fast on the average, one of them
+// slower by over 2 % (3 %).
 int64_t qgemm_dense_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M < 1024 || M > (1 << 30) || N < 256 || N > (1 << 30) || K < 1024 || K > (1 << 20) || K % BK || N % 8) return 0;
-    if (M * N < (K < 2048 ? 20000000 : M < 1280 ? 11500000 : 1 << 23)) return 0;
+    if (M < 1280 && K > 8192) return 0;
+    if (M * N < (K < 1536 ? 26000000 : K < 2048 ? 20000000 : M < 1280 ? 11500000 : 1 << 23)) return 0;
     const int64_t row = K * 2;
     int64_t rows = N;
     if (rows * row > WS_MAX_BYTES) rows = WS_MAX_BYTES / row / 256 * 256;   // whole 256-column tiles at a time
@@ -412,7 +440,7 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
     if ((bits != 4 && bits != 8) || (swiglu_half && N != 2 * swiglu_half)) return SC_EUNSUPPORTED;
     if (!wide_rows(y, N, swiglu_half)) return SC_EUNSUPPORTED;
     if (device_info().max_lds_per_block < 2 * (BM + 256) * ROW_BYTES) return SC_EUNSUPPORTED;
-    const int rows = (int)(need / ((int64_t)K * 2));
+    int rows = (int)(need / ((int64_t)K * 2));
     DenseArgs a;
     a.x = x; a.w = static_cast<const uint16_t *>(ws); a.bias = bias; a.y = y;
     a.M = M; a.K = K;
@@ -420,6 +448,17 @@ int launch_qgemm_dense(const uint16_t *x, const uint32_t *wq, const uint16_t *s,
     a.swiglu_i = swiglu_half;
     a.mt = (M + BM - 1) / BM;
     a.nt = a.tiles = 0;
+    if (rows < N) {
+        // Several chunks of columns: whole rounds of wide tiles each (W4 1854 x 13120 x 11456,
+        // 620 us on the fused GEMM, two chunks of the largest size 796, so 546).  Where the
+        // chunks' rounds still come to much more than the whole product's, the fused GEMM
+        // (1033 x 25280 x 11200, three chunks of 0.9, 0.9 and 0.7 rounds for 2: 663 -> 801).
+        const int64_t cus = device_info().num_cus, full = a.mt * (rows / 256) / cus;
+        if (full * cus / a.mt > 0) rows = (int)(full * cus / a.mt * 256);
+        int64_t cost = 0;
+        for (int n0 = 0; n0 < N; n0 += rows) cost += plan_dense(a.mt, N - n0 < rows ? N - n0 : rows).cost;
+        if (100 * cost > 115 * plan_dense(a.mt, N).cost) return SC_EUNSUPPORTED;
+    }
     for (int n0 = 0; n0 < N; n0 += rows) {
         const int nc = N - n0 < rows ? N - n0 : rows;
         const dim3 grid((unsigned)((nc + 3) / 4)), block(256);

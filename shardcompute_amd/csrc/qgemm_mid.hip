@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             if (m >= M) continue;
             uint32_t o[4] = {cvt_pk_bf16(acc[i][0][0], acc[i][0][1]), cvt_pk_bf16(acc[i][0][2], acc[i][0][3]),
                              cvt_pk_bf16(acc[i][1][0], acc[i][1][1]), cvt_pk_bf16(acc[i][1][2], acc[i][1][3])};
-            store_cols8<SWIGLU>(o, a.y + (size_t)m * a.ldy, n, n, N, a.bias != nullptr, bb);
+            store_cols8<false, SWIGLU>(o, a.y + (size_t)m * a.ldy, n, n, N, a.bias != nullptr, bb);
         }
     };
     if (a.swiglu_i) store(std::true_type{});

@@ -28,17 +28,17 @@ def _inputs(M, N, K, bits, seed):
     return x, wq, s, b, bias, ref, acc
 
 
-# rows and widths at the edges of the 256 x 256 and 256 x 128 tiles, stages of odd number, a last partial round as narrow tiles (12 x 43 wide tiles),
-# weights in two column chunks (N K above 2^27), the smallest products taken
-SHAPES = [(1280, 6592, 1088, 4), (1281, 15880, 1024 + 576, 8), (2048, 4096, 4096, 4), (2049, 4104, 2048, 8),
-          (2815, 11008, 2112, 4), (1030, 34000, 4096, 8), (40000, 512, 1024, 4)]
+# (256 CUs) the smallest products taken at each line of the size rule, ragged rows and columns,
+# stages of odd number, narrow tiles alone, wide ones alone (two rounds), a round of wide ones
+# and the last columns narrow, weights in two column chunks (N K above 2^27), many row tiles
+SHAPES = [(1280, 6560, 2048, 4), (1024, 11232, 2048, 8), (1600, 12504, 1536, 4), (1300, 20008, 1024, 8),
+          (1281, 15880, 1024 + 576, 8), (2048, 4096, 4096, 4), (2049, 4104, 2048, 8), (2815, 11008, 2112, 4),
+          (2041, 11272, 2112, 4), (2048, 28672, 1024, 8), (1030, 34000, 4096, 8), (51000, 512, 1024, 4)]
 
 
 @pytest.mark.parametrize("M,N,K,bits", SHAPES)
 def test_dense_against_reference(device, M, N, K, bits):
-    if not _lib.load().sc_qmm_workspace_bytes(M, N, K):
-        # below the size rule the same call runs the fused GEMM
-        assert M * N < 20000000 and K < 2048
+    assert _lib.load().sc_qmm_workspace_bytes(M, N, K) > 0
     print(f"dense M={M} N={N} K={K} bits={bits}", flush=True)
     x, wq, s, b, bias, ref, acc = _inputs(M, N, K, bits, M + N)
     y = _lib.qmm(x, wq, s, b, bits=bits)
@@ -82,10 +82,16 @@ def test_workspace_forms(device):
         assert not bad.any(), (y_off, ws_off, ws_bytes)
 
 
+@pytest.mark.parametrize("M,N,K", [(1279, 6560, 2048), (1280, 6552, 2048), (1023, 32768, 4096), (1024, 11224, 2048),
+                                   (1279, 16384, 8256), (1600, 12496, 1536), (1300, 19992, 1024), (4096, 4096, 960)])
+def test_below_the_size_rule_no_workspace(device, M, N, K):
+    assert _lib.load().sc_qmm_workspace_bytes(M, N, K) == 0
+
+
 def test_rows_of_element_stores_take_the_fused_gemm(device):
     """Widths that are no multiple of 8 want no workspace (2-byte stores cost the dense kernel
     more than it gains on most of them) and give the fused GEMM's bits."""
-    M, N, K, bits = 1300, 16001, 1088, 4
+    M, N, K, bits = 1300, 16001, 1600, 4
     assert _lib.load().sc_qmm_workspace_bytes(M, N, K) == 0 < _lib.load().sc_qmm_workspace_bytes(M, N - 1, K)
     x, wq, s, b, bias, _, _ = _inputs(M, N, K, bits, 3)
     assert torch.equal(_lib.qmm(x, wq, s, b, bias=bias, bits=bits),

@@ -59,7 +59,6 @@ struct FaGeo {
     static constexpr int LDS = FA_NST * STAGE;                   // 64 or 32 KB
     static constexpr int KSTEPS = D / 16;                        // 16-dim steps of S^T
     static constexpr int DB = D / 32;                            // 32-dim blocks of O^T
-    static constexpr int KROWS_PI = 1024 / KROW;                 // key rows of a DMA instruction
     static constexpr int DMA = KTILE / 1024 / 4;                 // K (and Vt) DMA instructions per wave
     // the growth of a column's maximum (log2) that moves it.  head_dim 64 rescales few
     // registers and always moves it: the largest probabilities then lie just below 1, where
@@ -174,9 +173,10 @@ attn_prefill_kernel(FaArgs a) {
 #pragma unroll
         for (int qq = 0; qq < Gm::DMA; ++qq) {
             const int qi = Gm::DMA * w + qq;
-            constexpr int CPR = Gm::KROW / 16;             // chunks of a key row
-            const int r = Gm::KROWS_PI * qi + lane / CPR;
-            const int c = fa_kpos<D>(r, lane % CPR);
+            // key row, chunk.  Shifts and masks: written as lane / 16 and lane % 16 the
+            // head_dim-128 copies took 8 registers more and 1-7 % longer
+            const int r = D == 128 ? 4 * qi + (lane >> 4) : 8 * qi + (lane >> 3);
+            const int c = D == 128 ? (lane & 15) ^ (fa_swap23(r) & 15) : (lane & 7) ^ ((r >> 1) & 7);
             const int key = min(kb + r, a.T_cap - 1);
             dma::dma16s(kbase, (uint32_t)(key * Gm::KROW + 16 * c), kl + 1024 * qi);
         }
@@ -296,10 +296,7 @@ attn_prefill_kernel(FaArgs a) {
             m = bm;
         }
         const float nms = -m * sc;
-        // the probabilities, packed to bf16 in pairs; their sum stays in fp32
         float ps = 0.f;
-        uint32_t pk[2][8];
-        float phold = 0.f;
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
@@ -314,9 +311,8 @@ attn_prefill_kernel(FaArgs a) {
                 } else {
                     p = __builtin_amdgcn_exp2f(fmaf(sacc[kh][r], sc, nms));
                 }
+                sacc[kh][r] = p;
                 ps += p;
-                if (r & 1) pk[kh][r >> 1] = cvt_pk_bf16(phold, p);
-                phold = p;
             }
         lsum = lsum * alpha + ps;
         // rescale O^T only when some column's maximum moved (wave-uniform test)
@@ -332,8 +328,11 @@ attn_prefill_kernel(FaArgs a) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
-            const int kh = s4 >> 1, p0 = 4 * (s4 & 1);
-            const bf16x8_t pb = as_bf16x8(pk[kh][p0], pk[kh][p0 + 1], pk[kh][p0 + 2], pk[kh][p0 + 3]);
+            const int kh = s4 >> 1, r0 = 8 * (s4 & 1);
+            const bf16x8_t pb = as_bf16x8(cvt_pk_bf16(sacc[kh][r0], sacc[kh][r0 + 1]),
+                                          cvt_pk_bf16(sacc[kh][r0 + 2], sacc[kh][r0 + 3]),
+                                          cvt_pk_bf16(sacc[kh][r0 + 4], sacc[kh][r0 + 5]),
+                                          cvt_pk_bf16(sacc[kh][r0 + 6], sacc[kh][r0 + 7]));
             const int c = 4 * kh + 2 * (s4 & 1) + lh;
             // cache slots at or past T may hold anything, NaN included: their zero
             // probabilities must not meet them, so the V pieces of the block that

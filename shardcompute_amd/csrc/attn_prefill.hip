@@ -124,7 +124,8 @@ attn_prefill_kernel(FaArgs a) {
     // per CU) are resident together, workgroup p beside p + pair_half in dispatch
     // order, so that round pairs rank j with rank 2 pair_half - 1 - j and each CU
     // gets about the same number of key blocks (a heuristic on dispatch order: any
-    // order gives the same results)
+    // order gives the same results).  Head_dim 64 without a mask has a third beside
+    // them, the ranks that follow in order
     int rank = (int)blockIdx.x;
     if (a.pair_half > 0 && rank < 2 * a.pair_half && rank >= a.pair_half) rank = 3 * a.pair_half - 1 - rank;
     const int nbh = (int)(gridDim.x / a.nqb);             // B * Hkv
@@ -413,8 +414,8 @@ static int launch_fa(const FaArgs &f, long wgs, hipStream_t stream) {
 // Launches attn_prefill_kernel when the shape suits it (head_dim 128 or 64, the GQA ratio
 // dividing 128, 16-byte aligned Vt, at least 128 / R new positions: one workgroup's
 // columns, a positive scale) and returns SC_OK; returns 1, launching nothing, when it
-// does not.  The choice does not depend on the batch size, so that a sequence's result is the same
-// alone and in a batch (every column's arithmetic is its own).  The caller has
+// does not.  At head_dim 128 the choice does not depend on the batch size, so that a sequence's
+// result is the same alone and in a batch (every column's arithmetic is its own).  The caller has
 // checked the shape, strides and pointers as launch_attention does.  mask / ms: the
 // additive mask and its strides (b, h, s, t), or null.
 int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, const uint16_t *vt, long T_cap,
@@ -426,14 +427,20 @@ int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, co
     // for a positive scale whose reciprocal is a normal number.  Any other scale (zero,
     // negative, NaN, the ends of the range) is attn_kernel's, which scales the scores first.
     if (!(scale >= 1e-30f && scale <= 1e30f)) return 1;
-    // head_dim 64: few query rows over many keys stay on attn_kernel, which splits the keys
-    // over workgroups (a workgroup here takes ~1 us per 64 keys).  Measured, one sequence,
-    // 32 q heads on 4 kv heads, attn_kernel -> here: 128 positions after 1500 16 -> 26 us,
-    // 192 24 -> 27, 256 25 -> 28, 384 47 -> 29; 384 after 300 26 -> 14, 64 after 300
-    // 14 -> 11; 8 heads of their own: 1024 after 1500 34 -> 38, 1024 after 300 25 -> 23; 701
-    // positions of 3 sequences 84 -> 19, 2048 of one 163 -> 37.  By the capacity and not
-    // the length, which only the device knows.
-    if (D == 64 && S * H < 12288 && T_cap > 512) return 1;
+    // head_dim 64: attn_kernel's workgroups (16 columns, the keys over 4 waves and, with few of
+    // them, over key ranges) walk the keys faster than one here (~1 us per 64 keys, with a mask
+    // ~2), so it stays while they are at most two rounds of the CUs, with a mask four (two where
+    // the cache is short).  Measured, us, attn_kernel -> here, no mask: 32 heads on 4 of one
+    // sequence, 209 positions (418 workgroups) 7.8 -> 8.2, 295 (590) 12.9 -> 9.2, 1028 45 -> 19;
+    // 4 heads of their own, 128 after 259 (32) 8.1 -> 11.4; 8 sequences of 32 heads on 8, 62
+    // (1000) 11.5 -> 7.1; a mask: 128 after 263 of 4 heads 10 -> 31, 447 of 16 heads on 1 (447)
+    // 16 -> 19, 1824 of 8 on 1 (912) 61 -> 65, 1028 of 32 on 4 (2056) 76 -> 40.  Over 403 sizes,
+    // masked and not, none is slower here, and 90-95 % of what the better kernel gives is taken.
+    if (D == 64) {
+        const long Pw = 16 / (R < 16 ? R : 16), cus = device_info().num_cus;
+        const long attn_wgs = B * Hkv * ((R + 15) / 16) * ((S + Pw - 1) / Pw);
+        if (attn_wgs <= (mask && T_cap > 128 ? 4 : 2) * cus) return 1;
+    }
     if (T_cap > (1L << 22)) return 1;    // staging offsets within one (b, kv head) slab are 32-bit
     const long nqb = (S + FA_COLS / R - 1) / (FA_COLS / R);
     const long wgs = B * Hkv * nqb;

@@ -1,9 +1,10 @@
-"""Prefill attention at head_dim 64 on the 128-column kernel against float64: positions at the
-edges of a workgroup's columns (128 / R positions), GQA ratios 8, 4 and 1, cached prefixes,
-garbage past the length, an additive mask, and both sides of the rule that keeps few query
-rows over a large cache on the key-splitting kernel.
+"""Prefill attention at head_dim 64 against float64, on the 128-column kernel and on either
+side of the rule that keeps the key-splitting kernel where its workgroups are few: positions
+at the edges of a workgroup's columns (128 / R positions), GQA ratios 1 to 32, cached
+prefixes, several 64-key blocks, garbage past the length, an additive mask.
 
-The bound is the attention's: bf16 probabilities and outputs, max |y - ref| <= 1e-2 max |ref|."""
+The bound is the attention's, bf16 probabilities and outputs, for each row by itself:
+|y - ref| <= 1e-2 |ref| in the 2-norm (probabilities and outputs each rounded by 2^-9 rms)."""
 import math
 
 import pytest
@@ -31,9 +32,15 @@ def _reference(q, k, v, past, mask):
     return out
 
 
-# (B, S, H, Hkv, past, T_cap): the last two on either side of S H = 12288 with a large cache
+# (B, S, H, Hkv, past, T_cap).  The first block runs on the key-splitting kernel (256 CUs: at
+# most 512 workgroups of 16 columns there, with a mask over more than 128 slots 1024), the
+# others on the 128-column one, those marked so without a mask only
 CASES = [(1, 16, 32, 4, 0, 32), (2, 17, 32, 4, 47, 96), (1, 33, 16, 4, 0, 64), (2, 129, 4, 4, 5, 160),
-         (1, 100, 8, 1, 300, 512), (3, 200, 32, 4, 0, 224), (1, 383, 32, 4, 400, 1024), (1, 385, 32, 4, 400, 1024)]
+         (1, 100, 8, 1, 300, 512), (1, 256, 32, 4, 400, 1024),
+         (1, 257, 32, 4, 400, 1024), (2, 129, 32, 32, 5, 160), (1, 385, 32, 4, 400, 1024),      # no mask
+         (17, 16, 32, 4, 0, 32), (16, 17, 32, 4, 47, 96), (3, 200, 32, 4, 0, 224), (1, 517, 32, 4, 0, 544),
+         (1, 515, 32, 4, 133, 672), (4, 129, 32, 32, 5, 160), (8, 70, 32, 8, 7, 96), (2, 530, 16, 1, 3, 544),
+         (1, 520, 32, 1, 0, 544)]
 
 
 @pytest.mark.parametrize("B,S,H,Hkv,past,T_cap", CASES)
@@ -62,7 +69,7 @@ def test_prefill_attention_head_dim_64(device, B, S, H, Hkv, past, T_cap, masked
                      None if mask is None else mask[:, 0])
     got = out.view(B, S, H, D).transpose(1, 2).double()
     assert torch.isfinite(got).all()
-    assert (got - ref).abs().max() <= 1e-2 * ref.abs().max()
+    assert ((got - ref).norm(dim=-1) <= 1e-2 * ref.norm(dim=-1)).all()
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -72,22 +79,22 @@ def test_prefill_softmax_sum_is_fp32(device, D, masked):
     (no running maximum), so the result is known to its last bit but for the few elements
     whose probabilities lie within the scores' fp32 error (~2^-20) of a bf16 rounding
     boundary, ~1e-3 of them; a sum of the rounded values moves 4-5 % of them."""
-    S, H, past = 40, 8, 24
+    B, S, H, past = 30, 40, 8, 24
     T = past + S
     g = torch.Generator(device="cuda")
     g.manual_seed(D)
-    q = torch.randn((S, H * D), generator=g, device="cuda").to(torch.bfloat16)
-    kc = torch.randn((1, 1, T, D), generator=g, device="cuda").to(torch.bfloat16)
-    vt = torch.randn((1, 1, D, T), generator=g, device="cuda").to(torch.bfloat16)
+    q = torch.randn((B * S, H * D), generator=g, device="cuda").to(torch.bfloat16)
+    kc = torch.randn((B, 1, T, D), generator=g, device="cuda").to(torch.bfloat16)
+    vt = torch.randn((B, 1, D, T), generator=g, device="cuda").to(torch.bfloat16)
     mask = torch.randn((1, 1, 1, T), generator=g, device="cuda") if masked else None
     cnt = torch.tensor([past, 0], dtype=torch.int32, device="cuda")
-    out = _lib.attention(q, 1, S, H, 1, D, kc, vt, cnt, 1 / math.sqrt(D), mask=mask, n_keys=T).view(S, H, D)
-    hidden = torch.arange(T, device="cuda")[None] > torch.arange(past, T, device="cuda")[:, None]
-    s = q.view(S, H, D).transpose(0, 1).double() @ kc[0, 0].double().T.contiguous() / math.sqrt(D)
+    out = _lib.attention(q, B, S, H, 1, D, kc, vt, cnt, 1 / math.sqrt(D), mask=mask, n_keys=T).view(B, S * H, D)
+    limit = torch.arange(past, T, device="cuda").repeat_interleave(H)
+    s = torch.bmm(q.view(B, S * H, D).double(), kc[:, 0].double().transpose(1, 2).contiguous()) / math.sqrt(D)
     if masked:
-        s = s + mask[0].double()
-    s = s.masked_fill(hidden, -math.inf)
+        s = s + mask[0, 0].double()
+    s = s.masked_fill(torch.arange(T, device="cuda") > limit[:, None], -math.inf)
     p = torch.exp(s - s.amax(-1, keepdim=True))
-    o = p.float().to(torch.bfloat16).double() @ vt[0, 0].double().T.contiguous()
+    o = torch.bmm(p.float().to(torch.bfloat16).double(), vt[:, 0].double().transpose(1, 2).contiguous())
     exact = (o / p.sum(-1, keepdim=True)).float().to(torch.bfloat16)
-    assert (out.transpose(0, 1) != exact).double().mean() <= 0.01
+    assert (out != exact).double().mean() <= 0.01

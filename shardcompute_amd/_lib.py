@@ -233,7 +233,10 @@ def qmm(x, wq, scales, biases, bias=None, bits=4, group_size=64, path=PATH_AUTO,
     """y = bf16(x @ dequant(wq, scales, biases)^T) (+ bias), x [..., K] -> [..., N].
 
     ``no_alloc``: call ``sc_qmm_bf16_noalloc`` (the library allocates nothing;
-    pass ``out`` too for a call that allocates nothing at all).
+    pass ``out`` too for a call that allocates nothing at all).  The result is that of the
+    plain call bit for bit below 1024 rows, unless the split-K partials exceed the library's
+    fixed scratch; from there on the plain call may take a workspace and the dense GEMM,
+    this one never does.
     ``band_plan``: (waves, ksplit) pins the band kernel's plan (``sc_qmm_bf16_band``;
     0 = automatic), for measurements."""
     lib = load()

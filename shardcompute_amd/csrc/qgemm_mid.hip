@@ -259,13 +259,11 @@ static int launch_mid_t(const MidArgs &a, int splits, hipStream_t stream) {
     return SC_OK;
 }
 
-// K splits of a product of `tiles` tiles over nb scale/bias blocks
+// K splits of a product of `tiles` tiles, a quarter of the CUs at most, over nb >= 8
+// scale/bias blocks: about one workgroup a CU, at least 16 stages each
 static int mid_splits(int64_t tiles, int nb) {
-    const int cus = device_info().num_cus;
-    int ks = 1;
-    if (tiles * 2 <= cus) ks = (int)(cus / tiles);         // about one workgroup a CU
-    if (ks > nb / 2) ks = nb / 2;                          // at least 16 stages each
-    if (ks < 1) ks = 1;
+    int ks = (int)(device_info().num_cus / tiles);
+    if (ks > nb / 2) ks = nb / 2;
     const int bps = (nb + ks - 1) / ks;
     return (nb + bps - 1) / bps;
 }
@@ -296,10 +294,10 @@ int launch_qgemm_mid(const uint16_t *x, const uint32_t *wq, const uint16_t *s, c
     // 34 -> 28, 768 rows (96) 44 -> 46; 4096 -> 6144 170 rows (96) 34 -> 35.
     if (tiles > (K < 4096 ? device_info().num_cus : device_info().num_cus / 4)) return SC_EUNSUPPORTED;
     a.tiles = (int)tiles;
-    // Only the products that qgemm.hip splits too (its wide tiles fill at most a quarter of
-    // the CUs, K >= 4096) split K, because the partials live in the library's scratch.
-    const int64_t tiles256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-    int splits = 4 * tiles256 <= device_info().num_cus && a.G >= 64 ? mid_splits(tiles, a.G / 8) : 1;
+    // K is split from 4096 on, where qgemm.hip splits each of these products too (its 256-wide
+    // tiles are no more than these, a quarter of the CUs), because the partials live in the
+    // library's scratch.  No-alloc partials beyond the fixed array: K whole.
+    int splits = K >= 4096 ? mid_splits(tiles, a.G / 8) : 1;
     const size_t need = (size_t)splits * M * N;
     if (splits > 1 && no_alloc && need * sizeof(float) > (size_t)SC_QMM_NOALLOC_SCRATCH_BYTES) splits = 1;
     if (splits == 1) return bits == 4 ? launch_mid_t<4>(a, 1, stream) : launch_mid_t<8>(a, 1, stream);

@@ -45,3 +45,20 @@ def test_mid_swiglu_equals_product_then_gate(device, M, I, K, bits, with_bias):
     bias = bias if with_bias else None
     act, _ = _lib.qmm_swiglu(x, wq, s, b, bias=bias, bits=bits)
     assert torch.equal(act, _lib.silu_mul(_lib.qmm(x, wq, s, b, bias=bias, bits=bits)))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K,equal", [(200, 304, 4096, True), (333, 2048, 5632, False), (300, 1000, 2048, True)])
+def test_mid_without_allocation(device, bits, M, N, K, equal):
+    """Split-K partials that fit the allocation-free array (4 MiB): sc_qmm_bf16's bits; partials
+    that do not (4 x 333 x 2048 floats): K whole, against the reference."""
+    print(f"mid noalloc M={M} N={N} K={K} W{bits}", flush=True)
+    x, wq, s, b, bias = _inputs(M, N, K, bits)
+    y = _lib.qmm(x, wq, s, b, bias=bias, bits=bits)
+    yn = _lib.qmm(x, wq, s, b, bias=bias, bits=bits, no_alloc=True)
+    assert torch.equal(y, yn) == equal
+    w = _lib.dequantize(wq, s, b, bits=bits).double()
+    p = x.double() @ w.T
+    ref = p + bias.double()
+    acc = 8 * math.sqrt(K) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert not ((yn.double() - ref).abs() > 2.0 ** -8 * (ref.abs() + p.abs()) + acc).any()

@@ -107,7 +107,8 @@ def test_qmm_swiglu_matches_unfused(device, M, I, K, bits, norm):
 @pytest.mark.parametrize("M,bits", [(2048, 4), (2048, 8)])
 def test_qmm_swiglu_prefill_shape_matches_unfused(device, M, bits):
     # the Llama-3-8B gate|up at a 2048-token prefill: wide tiles plus the 128-wide
-    # launch for the partial last round, both pairing gate and up columns
+    # launch for the partial last round, both pairing gate and up columns, on the dense GEMM
+    # (the binding brings its workspace) and on the GEMM of the entry without one
     rng = np.random.default_rng(M + bits)
     I, K = 14336, 4096
     wq, s, b = _weights(rng, 2 * I, K, bits)
@@ -118,6 +119,13 @@ def test_qmm_swiglu_prefill_shape_matches_unfused(device, M, bits):
     act2 = _lib.silu_mul(_lib.qmm(xd, *W, bits=bits))
     torch.cuda.synchronize()
     assert torch.equal(act, act2)
+    act.fill_(float("nan"))
+    gu = torch.empty((M, 2 * I), dtype=torch.bfloat16, device="cuda")
+    P = _lib._ptr
+    assert _lib.load().sc_qmm_swiglu_bf16(P(xd), None, None, 1e-5, None, None, *map(P, W), None, P(act), P(gu), M, I, K,
+                                          bits, 64, _lib._stream(xd)) == 0
+    act3 = _lib.silu_mul(_lib.qmm(xd, *W, bits=bits, path=_lib.PATH_GEMM))
+    assert torch.equal(act, act3)
 
 
 @pytest.mark.parametrize("M,bits", [(9, 4), (16, 8), (32, 4), (200, 4), (1100, 8)])

@@ -251,13 +251,15 @@ int sc_decode_head_bf16(const uint16_t *x, const uint16_t *residual_or_null, con
  * xn = RMSNorm(x + residual) when norm_weight_or_null is given (xn_out and, with a
  * residual, h_out receive xn and x + residual as for sc_qmm_rmsnorm_bf16).  The
  * decode GEMV (M <= 8) pairs gate row i with up row I + i inside one tile and writes
- * act [M, I] directly; at 9-160 rows (band kernel, K a multiple of 512, chosen by
- * shape up to 32 rows; else the split-K GEMV) the split-K pass rounds gate and up to bf16 (bias after
- * rounding) and writes act [M, I]; above that the GEMM pairs gate and up columns in its tiles
- * and writes act itself (I a multiple of 16).  gate_up_scratch [M, 2I] is required but
- * used only where none of these applies: then the product goes there and the
- * standalone sc_silu_mul_bf16 follows (the same values).  Outputs must not overlap
- * the inputs.
+ * act [M, I] directly, its sums in another order than the plain product's; at 9-160 rows
+ * (band kernel, K a multiple of 512, chosen by shape up to 32 rows; else the split-K GEMV) the
+ * split-K pass rounds gate and up to bf16 (bias after rounding) and writes act [M, I]; above
+ * that the GEMM pairs gate and up columns in its tiles and writes act itself (I a multiple of
+ * 16).  gate_up_scratch [M, 2I] is required and used where none of these applies, also where
+ * K is in one piece at 9-160 rows: then the product goes there and the standalone
+ * sc_silu_mul_bf16 follows.  From 9 rows on act is that of the plain product and its
+ * activation bit for bit, and the library's split-K scratch is taken where the plain product
+ * takes it.  Outputs must not overlap the inputs.
  * Replaces ParallelMLP.forward's gate/up projections and activation
  * (src/shardcompute/parallel/mlp.py:241-245), after the post-attention layernorm
  * (transformer.py:249-250).

@@ -427,19 +427,30 @@ int launch_attn_prefill(const uint16_t *q, long q_stride, const uint16_t *kc, co
     // for a positive scale whose reciprocal is a normal number.  Any other scale (zero,
     // negative, NaN, the ends of the range) is attn_kernel's, which scales the scores first.
     if (!(scale >= 1e-30f && scale <= 1e30f)) return 1;
-    // head_dim 64: attn_kernel's workgroups (16 columns, the keys over 4 waves and, with few of
-    // them, over key ranges) walk the keys faster than one here (~1 us per 64 keys, with a mask
-    // ~2), so it stays while they are at most two rounds of the CUs, with a mask four (two where
-    // the cache is short).  Measured, us, attn_kernel -> here, no mask: 32 heads on 4 of one
-    // sequence, 209 positions (418 workgroups) 7.8 -> 8.2, 295 (590) 12.9 -> 9.2, 1028 45 -> 19;
-    // 4 heads of their own, 128 after 259 (32) 8.1 -> 11.4; 8 sequences of 32 heads on 8, 62
-    // (1000) 11.5 -> 7.1; a mask: 128 after 263 of 4 heads 10 -> 31, 447 of 16 heads on 1 (447)
-    // 16 -> 19, 1824 of 8 on 1 (912) 61 -> 65, 1028 of 32 on 4 (2056) 76 -> 40.  Over 403 sizes,
-    // masked and not, none is slower here, and 90-95 % of what the better kernel gives is taken.
+    // head_dim 64: attn_kernel's workgroups (16 columns, the keys over 4 waves) walk the keys
+    // faster than one here (~1 us per 64 keys, with a mask ~2), so it stays while they are about
+    // two rounds of the CUs.  Under one round it also splits the keys over workgroups and merges
+    // them in a second launch (8-12 us in all), which a cache of a few blocks beats here.  With a
+    // mask it stays up to four rounds, two where there are few positions or slots, one more where
+    // every column has a mask row of its own (2053 positions of 8 heads 104 -> 118).  Measured, us,
+    // attn_kernel -> here, no mask: 32 heads on 4 of one sequence, 209 positions (418 workgroups)
+    // 7.8 -> 8.2, 295 (590) 12.9 -> 9.2, 1028 45 -> 19; 4 heads of their own, 128 after 259 (32)
+    // 8.1 -> 11.4; 8 of 3 sequences, 150 in 320 slots (240) 11.9 -> 6.7; 8 sequences of 32 heads
+    // on 8, 62 (1000) 11.5 -> 7.1; a mask: 128 after 263 of 4 heads 10 -> 31, 447 of 16 heads on 1
+    // (447) 16 -> 19, 1867 of 8 on 1 (934) 61 -> 64, 1028 of 32 on 4 (2056) 76 -> 40.  Over 1590
+    // sizes, masked and not, up to 16000 cached positions, none is slower here by over 3 %, and
+    // 94-97 % of the better kernel's gain is taken.  By the capacity where the length would matter, which
+    // only the device knows.
     if (D == 64) {
         const long Pw = 16 / (R < 16 ? R : 16), cus = device_info().num_cus;
         const long attn_wgs = B * Hkv * ((R + 15) / 16) * ((S + Pw - 1) / Pw);
-        if (attn_wgs <= (mask && T_cap > 128 ? 4 : 2) * cus) return 1;
+        const long own = R == 1 ? cus : 0;                   // a mask row per column: a round more
+        const bool splits = attn_wgs < cus && T_cap > 128;
+        const bool take = mask ? attn_wgs > 4 * cus + own ||
+                                     (attn_wgs > 2 * cus + own && (S <= 256 || T_cap <= 128))
+                               : 16 * attn_wgs > 33 * cus ||
+                                     (splits && (T_cap + 63) / 64 <= 2 + 7 * attn_wgs / (2 * cus));
+        if (!take) return 1;
     }
     if (T_cap > (1L << 22)) return 1;    // staging offsets within one (b, kv head) slab are 32-bit
     const long nqb = (S + FA_COLS / R - 1) / (FA_COLS / R);

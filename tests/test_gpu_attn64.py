@@ -33,11 +33,14 @@ def _reference(q, k, v, past, mask):
 
 
 # (B, S, H, Hkv, past, T_cap).  The first block runs on the key-splitting kernel (256 CUs: at
-# most 512 workgroups of 16 columns there, with a mask over more than 128 slots 1024), the
-# others on the 128-column one, those marked so without a mask only
+# most 528 workgroups of 16 columns there, with a mask 1024, or 512 for up to 256 positions or
+# 128 slots, 256 more for a kv head per q head), the others on the 128-column one, those marked
+# so without a mask only (the last two of them: few workgroups there, which would split the
+# keys of a short cache)
 CASES = [(1, 16, 32, 4, 0, 32), (2, 17, 32, 4, 47, 96), (1, 33, 16, 4, 0, 64), (2, 129, 4, 4, 5, 160),
-         (1, 100, 8, 1, 300, 512), (1, 256, 32, 4, 400, 1024),
-         (1, 257, 32, 4, 400, 1024), (2, 129, 32, 32, 5, 160), (1, 385, 32, 4, 400, 1024),      # no mask
+         (1, 100, 8, 1, 300, 512), (1, 264, 32, 4, 400, 1024), (3, 150, 8, 8, 100, 352),
+         (1, 265, 32, 4, 400, 1024), (1, 385, 32, 4, 400, 1024), (2, 129, 32, 32, 5, 160),       # no mask
+         (3, 150, 8, 8, 0, 320), (2, 97, 16, 2, 60, 192),                                        # no mask
          (17, 16, 32, 4, 0, 32), (16, 17, 32, 4, 47, 96), (3, 200, 32, 4, 0, 224), (1, 517, 32, 4, 0, 544),
          (1, 515, 32, 4, 133, 672), (4, 129, 32, 32, 5, 160), (8, 70, 32, 8, 7, 96), (2, 530, 16, 1, 3, 544),
          (1, 520, 32, 1, 0, 544)]

@@ -452,7 +452,11 @@ def qmm_swiglu(x, wq, scales, biases, norm_weight=None, eps=1e-5, residual=None,
     if residual is not None:
         _rows(residual, K, "residual")
     act = x.new_empty((M, I)) if act_out is None else _rows(act_out, I, "act_out")
-    gu = x.new_empty((M, N)) if gate_up_scratch is None else _rows(gate_up_scratch, N, "gate_up_scratch")
+    gu = gate_up_scratch
+    if gu is not None:
+        _rows(gu, N, "gate_up_scratch")
+    if gu is None or gu.numel() < M * N:        # a scratch of fewer rows did where the kernel used none
+        gu = x.new_empty((M, N))
     ws, ws_bytes = _qmm_workspace(M, N, K, x.device)
     rc = lib.sc_qmm_swiglu_bf16_ws(_ptr(x), _ptr(residual), _ptr(norm_weight), float(eps), _ptr(h_out), _ptr(xn),
                                    _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(act), _ptr(gu), M, I, K,

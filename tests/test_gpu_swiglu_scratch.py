@@ -7,6 +7,9 @@ import subprocess
 import sys
 
 import pytest
+import torch
+
+from shardcompute_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +48,17 @@ def test_unsplit_swiglu_takes_no_scratch(device, M, I, K, bits):
                        capture_output=True, text=True, timeout=100, cwd=root)
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
     assert "captured ok" in p.stdout
+
+
+def test_scratch_of_fewer_rows_is_left_alone(device):
+    """gate_up_scratch is [rows, 2 I]; one of fewer rows is not written past its end (nor
+    before it): the binding takes its own."""
+    M, I, K, bits = 24, 512, 512, 4
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    x = torch.randn((M, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = _lib.quantize(torch.randn((2 * I, K), generator=g, device="cuda").mul_(0.02), bits=bits)
+    whole = torch.full((M, 2 * I), 7.0, dtype=torch.bfloat16, device="cuda")
+    act, _ = _lib.qmm_swiglu(x, *w, bits=bits, gate_up_scratch=whole[:3])
+    assert torch.equal(act, _lib.silu_mul(_lib.qmm(x, *w, bits=bits)))
+    assert (whole == 7.0).all()
